@@ -27,6 +27,7 @@ SOURCES = (
     "paged_decode.hip",
     "paged_decode_mfma.hip",
     "paged_prefill.hip",
+    "paged_prefill_f32.hip",
     "rope_append.hip",
     "read_probe.hip",
 )
@@ -52,9 +53,11 @@ COMMON_FLAGS = [
 # wave per SIMD) then lose the accumulator-register copies the allocator
 # otherwise places in every tile (MQA balanced split 29.7 -> 28.6 us); the
 # 16-head kernels already allocate VGPRs only (two waves per SIMD) and are
-# unchanged.
+# unchanged. The fp32 prefill kernels gain a wave per SIMD by it (54.5 ->
+# 51.4 us at head_dim 64).
 SOURCE_FLAGS = {
     "paged_prefill.hip": ["-fno-honor-nans"],
+    "paged_prefill_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "paged_decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

@@ -27,85 +27,21 @@
 //    exactly the P operand of a 32-deep PV MFMA; its V^T operand is two
 //    ds_read_b64_tr_b16 of the staged tile.
 //
-//  * VALU (every other dtype / head_dim <= 256 / block size):
-//    paged_prefill_scalar_kernel, one wave per (request, head, row), keys in
-//    sequence, fp32 online softmax.
+//  * every other dtype / head_dim / block size: paged_prefill_f32_kernel
+//    (paged_prefill_f32.hip, fp32 matrix cores) up to head_dim 256; wider
+//    16-bit rows run paged_prefill_scalar_kernel, one wave per (request,
+//    head, row), keys in sequence, fp32 online softmax.
 //
 // Blocks whose table entry lies outside [0, num_blocks) are masked as in the
 // decode kernels; no load ever leaves the cache.
 #include "ikl_common.h"
 #include "mfma_ops.h"
 #include "paged_attn.h"
+#include "paged_prefill.h"
 
 namespace ikl {
 
-struct PrefillParams {
-  const char *q;
-  int64_t q_sb, q_sh, q_st;  // elements
-  const char *kc;
-  const char *vc;
-  int64_t k_sb, k_st, k_sh;
-  int64_t v_sb, v_st, v_sh;
-  const void *tables;
-  int64_t t_sb;
-  int64_t table_width;
-  const void *starts;
-  const void *lens;
-  char *out;
-  int64_t o_sb, o_sh, o_st;
-  int64_t batch;
-  int64_t width;       // query rows per request (T)
-  int64_t num_blocks;
-  int64_t cap_tokens;  // table_width * block_size
-  int64_t row_blocks;  // workgroups per (request, kv head) of the MFMA kernel
-  int64_t bh_pad;      // batch * num_kv_heads rounded up to a multiple of 8
-  int32_t stream_major;  // each XCD takes its (request, kv head) prefixes one after another
-  int32_t num_heads;
-  int32_t num_kv_heads;
-  int32_t heads_per_kv;
-  int32_t head_dim;
-  int32_t block_size;
-  int32_t bs_shift;  // log2(block_size) or -1
-  int32_t table_i64;
-  int32_t idx_i64;   // starts / lens element type
-  float scale_log2;  // scale * log2(e)
-  // FP8 KV cache: E4M3 codes, one fp32 scale per (token, head) row in
-  // k_scale / v_scale [blocks, kv heads, block_size]
-  int32_t kv_fp8;
-  const float *k_scale;
-  const float *v_scale;
-  int64_t s_sb, s_sh;  // elements
-};
-
 namespace {
-
-__device__ inline int64_t pf_index(const void *base, int64_t i, int i64) {
-  return i64 ? load_index<int64_t>(base, i) : load_index<int32_t>(base, i);
-}
-
-// Block-table entry (b, lb), or -1 when it is outside the table or names a
-// block outside the cache.
-__device__ inline int pf_block(const PrefillParams &p, int64_t b, int64_t lb) {
-  if (lb < 0 || lb >= p.table_width) return -1;
-  const int64_t e = pf_index(p.tables, b * p.t_sb + lb, p.table_i64);
-  return e >= 0 && e < p.num_blocks ? (int)e : -1;
-}
-
-// Prefill range of request b: start (clamped to [0, end]), end (clamped to
-// [0, cap_tokens]) and the number of attending rows (<= width).
-__device__ inline void pf_range(const PrefillParams &p, int64_t b, int64_t *start, int64_t *end, int64_t *rows) {
-  int64_t e = pf_index(p.lens, b, p.idx_i64);
-  e = e < 0 ? 0 : (e < p.cap_tokens ? e : p.cap_tokens);
-  int64_t s = pf_index(p.starts, b, p.idx_i64);
-  s = s < 0 ? 0 : (s < e ? s : e);
-  *start = s;
-  *end = e;
-  *rows = e - s < p.width ? e - s : p.width;
-}
-
-__device__ inline int64_t pf_logical(const PrefillParams &p, int64_t pos) {
-  return p.bs_shift >= 0 ? (pos >> p.bs_shift) : pos / p.block_size;
-}
 
 constexpr int PT = 32;     // keys per tile
 constexpr int PWAVES = 4;  // waves per workgroup
@@ -538,16 +474,10 @@ __global__ __launch_bounds__(64 * PWAVES) IKL_PREFILL_WAVES_ATTR void paged_pref
 
 // ------------------------------------------------------------------ VALU
 // One wave per (request, head, row). The lanes split the row's head_dim in
-// 4-byte granules (one fp32 or two 16-bit elements; up to 4 per lane), walk
+// 4-byte granules (two 16-bit elements; up to 4 per lane), walk
 // the keys in order and keep an fp32 online softmax in the log2 domain.
 template <typename Tag>
 struct granule;
-template <>
-struct granule<f32_tag> {
-  static constexpr int EB = 4, PER = 1;
-  __device__ static inline void unpack(uint32_t w, float *x) { x[0] = __uint_as_float(w); }
-  __device__ static inline uint32_t pack(const float *x) { return __float_as_uint(x[0]); }
-};
 template <>
 struct granule<bf16_tag> {
   static constexpr int EB = 2, PER = 2;
@@ -808,11 +738,17 @@ extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void
   } else {
     const int64_t blocks = a->batch * a->num_heads * a->query_width;
     if (blocks > 0x7fffffffLL) return fail(IKL_EINVAL, "ikl_paged_prefill_attention: launch too large");
-    const dim3 grid((unsigned)blocks);
-    if (a->dtype == IKL_BF16) paged_prefill_scalar_kernel<bf16_tag><<<grid, 64, 0, s>>>(p);
-    else if (a->dtype == IKL_F16) paged_prefill_scalar_kernel<f16_tag><<<grid, 64, 0, s>>>(p);
-    else paged_prefill_scalar_kernel<f32_tag><<<grid, 64, 0, s>>>(p);
-    err = hipGetLastError();
+    // The fp32 matrix cores wherever their kernel is compiled; 16-bit rows
+    // of 257-512 elements (fp32 rows end at 256) keep one wave per row: a
+    // 512-wide accumulator and its query would fill a wave's registers.
+    if (a->head_dim <= PREFILL_F32_MAX_DIM) {
+      err = launch_prefill_f32(p, a->dtype, s);
+    } else {
+      const dim3 grid((unsigned)blocks);
+      if (a->dtype == IKL_BF16) paged_prefill_scalar_kernel<bf16_tag><<<grid, 64, 0, s>>>(p);
+      else paged_prefill_scalar_kernel<f16_tag><<<grid, 64, 0, s>>>(p);
+      err = hipGetLastError();
+    }
   }
   if (err != hipSuccess) return fail(IKL_ELAUNCH, std::string("ikl_paged_prefill_attention: ") + hipGetErrorString(err));
   if (ev1 && hipEventRecord(ev1, s) != hipSuccess) return check_launch("ikl_paged_prefill_attention: event record");

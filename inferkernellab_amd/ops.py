@@ -874,7 +874,9 @@ class PreparedPagedPrefill:
         self._args = a
 
     def kernel_name(self) -> str:
-        return "paged_prefill_mfma_kernel" if self.path == "mfma_grouped" else "paged_prefill_scalar_kernel"
+        if self.path == "mfma_grouped":
+            return "paged_prefill_mfma_kernel"
+        return "paged_prefill_f32_kernel" if self.shape[-1] <= 256 else "paged_prefill_scalar_kernel"
 
     def __call__(self, query: torch.Tensor, layer: int = 0, *, out: torch.Tensor | None = None,
                  events=None) -> torch.Tensor:
