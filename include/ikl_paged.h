@@ -295,6 +295,30 @@ int ikl_hbm_read_probe(const void *buffer, int64_t bytes, void *sink, int64_t si
 #define IKL_ABI_VERSION 3
 int32_t ikl_abi_version(void);
 
+/* Findings of ikl_check_metadata, a bit each. */
+#define IKL_CHECK_LENGTH_POSITIVE 1u /* a context length <= 0 */
+#define IKL_CHECK_LENGTH_CAPACITY 2u /* a context length above table_width * block_size */
+#define IKL_CHECK_BLOCK_ID 4u        /* a table entry outside [0, num_blocks) */
+#define IKL_CHECK_LENGTH_MAX 8u      /* a context length above max_context */
+#define IKL_CHECK_PENDING 0xffffffffu
+
+/* Enqueues the value checks of triton_ops.py:439-457 over tables [batch,
+ * width] and lens [batch] (element strides; every table entry is checked,
+ * padding included; max_context 0 = no such bound) and returns how many
+ * words of `flags` the launch fills (1 .. num_flags), or a negative IKL_E*
+ * code (IKL_ELAUNCH while the stream is being captured: the result is read
+ * back). `flags`: pinned host memory the device can write, not touched by
+ * the caller until ikl_check_metadata_wait has returned for it. */
+int32_t ikl_check_metadata(const void *tables, int32_t table_type, int64_t table_stride_b, int64_t table_stride_w,
+                           const void *lens, int32_t lens_type, int64_t lens_stride, int64_t batch, int64_t width,
+                           int64_t block_size, int64_t num_blocks, int64_t max_context, uint32_t *flags,
+                           int32_t num_flags, void *stream);
+
+/* Waits for the `count` words of a check enqueued on `stream` (work enqueued
+ * after it is not waited for) and returns its findings, or a negative IKL_E*
+ * code when the launch failed. */
+int32_t ikl_check_metadata_wait(const uint32_t *flags, int32_t count, void *stream);
+
 /* KV append (in place). Slots outside [0, num_blocks*block_size) are skipped,
  * never written. Replaces append.py:69-106 / cache.py:156-189. */
 int ikl_append_kv(const ikl_append_args *args, void *stream);

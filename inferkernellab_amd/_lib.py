@@ -22,6 +22,8 @@ IKL_F16, IKL_BF16, IKL_F32, IKL_FP8_E4M3 = 0, 1, 2, 3
 IKL_I32, IKL_I64 = 0, 1
 IKL_OK, IKL_EINVAL, IKL_EUNSUPPORTED, IKL_ELAUNCH, IKL_EWORKSPACE = 0, -1, -2, -3, -4
 IKL_PATH_MHA_FALLBACK, IKL_PATH_SCALAR_GROUPED, IKL_PATH_MFMA_GROUPED = 0, 1, 2
+# findings of ikl_check_metadata
+IKL_CHECK_LENGTH_POSITIVE, IKL_CHECK_LENGTH_CAPACITY, IKL_CHECK_BLOCK_ID, IKL_CHECK_LENGTH_MAX = 1, 2, 4, 8
 # IKL_ABI_VERSION of the header these mirrors follow; load() refuses a
 # library that reports another
 IKL_ABI_VERSION = 3
@@ -30,6 +32,8 @@ EXPORTED_SYMBOLS = (
     "ikl_last_error",
     "ikl_version",
     "ikl_abi_version",
+    "ikl_check_metadata",
+    "ikl_check_metadata_wait",
     "ikl_append_kv",
     "ikl_paged_attention_workspace_size",
     "ikl_paged_attention_partition_size",
@@ -251,6 +255,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ikl_version.argtypes = []
     lib.ikl_abi_version.restype = _c_i32
     lib.ikl_abi_version.argtypes = []
+    lib.ikl_check_metadata.restype = _c_i32
+    lib.ikl_check_metadata.argtypes = [_c_ptr, _c_i32, _c_i64, _c_i64, _c_ptr, _c_i32, _c_i64, _c_i64, _c_i64,
+                                       _c_i64, _c_i64, _c_i64, _c_ptr, _c_i32, _c_ptr]
+    lib.ikl_check_metadata_wait.restype = _c_i32
+    lib.ikl_check_metadata_wait.argtypes = [_c_ptr, _c_i32, _c_ptr]
     lib.ikl_append_kv.restype = ctypes.c_int
     lib.ikl_append_kv.argtypes = [ctypes.POINTER(AppendArgs), _c_ptr]
     lib.ikl_paged_attention_workspace_size.restype = _c_i64

@@ -24,6 +24,7 @@ ARCH = "gfx950"
 SOURCES = (
     "abi.hip",
     "append_kv.hip",
+    "check_metadata.hip",
     "paged_decode.hip",
     "paged_decode_mfma.hip",
     "paged_prefill.hip",

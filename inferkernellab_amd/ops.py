@@ -24,7 +24,9 @@ without the built library or a GPU it raises ``RuntimeError``.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import threading
 
 import torch
 
@@ -116,12 +118,76 @@ def _as_index_tensor(value, device: torch.device) -> torch.Tensor:
     return value
 
 
+def _on_device(device: torch.device):
+    """Context with `device` current (nothing to switch where it is)."""
+    if device.index is None or torch.cuda.current_device() == device.index:
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
+
+
+_check_flags = threading.local()  # one pinned buffer a thread: a check is waited for before the next begins
+_CHECK_WORDS = 64
+_CHECK_MESSAGES = (  # in the order of triton_ops.py:439-457
+    (_lib.IKL_CHECK_LENGTH_POSITIVE, "context lengths must be positive"),
+    (_lib.IKL_CHECK_LENGTH_CAPACITY, "context length exceeds block table capacity"),
+    (_lib.IKL_CHECK_BLOCK_ID, "block table contains an invalid physical block id"),
+    (_lib.IKL_CHECK_LENGTH_MAX, "context length exceeds max_context_len"),
+)
+
+
+class _MetadataCheck:
+    """The value checks of block tables and context lengths, enqueued on the
+    current stream; ``wait`` raises what they found. The host prepares the
+    attention launch meanwhile. As a context manager it waits on leaving, so
+    that a finding is raised before any later error of the call."""
+
+    def __init__(self, block_tables, context_lens, layout, max_context_len):
+        self._lib = _require_backend()
+        flags = getattr(_check_flags, "words", None)
+        if flags is None:
+            flags = _check_flags.words = torch.empty(_CHECK_WORDS, dtype=torch.int32, pin_memory=True)
+        device = context_lens.device
+        with _on_device(device):
+            self._stream = torch.cuda.current_stream(device).cuda_stream
+            self._flags = flags.data_ptr()
+            self._count = self._lib.ikl_check_metadata(
+                block_tables.data_ptr(), _INDEX_TYPES[block_tables.dtype], block_tables.stride(0),
+                block_tables.stride(1), context_lens.data_ptr(), _INDEX_TYPES[context_lens.dtype],
+                context_lens.stride(0), block_tables.shape[0], block_tables.shape[1], layout.block_size,
+                layout.num_blocks, int(max_context_len or 0), self._flags, _CHECK_WORDS, self._stream)
+        _lib.check(min(self._count, 0), "check metadata")
+
+    def wait(self) -> None:
+        count, self._count = self._count, 0
+        if count <= 0:
+            return
+        found = self._lib.ikl_check_metadata_wait(self._flags, count, self._stream)
+        if found < 0:
+            _check_flags.words = None
+            _lib.check(found, "check metadata")
+        for bit, message in _CHECK_MESSAGES:
+            if found & bit:
+                raise ValueError(message)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        self.wait()
+        return False
+
+
+class _NoCheck(contextlib.nullcontext):
+    def wait(self) -> None:
+        pass
+
+
 def _validate_attention(query, cache, block_tables, context_lens, layer, validate_inputs,
                         max_context_len=None):
     """Checks of triton_ops.py:415-457, in the same order with the same
     messages, plus this library's ``max_context_len`` hint (a bound of
     ``context_lens`` that sizes the fixed-partition grid); returns the table
-    and length tensors."""
+    and length tensors and the value checks, enqueued but not waited for."""
     if query.ndim != 3 or query.device.type != "cuda":
         raise ValueError("query must be a GPU (torch 'cuda' device) tensor with shape [B,H,D]")
     if query.shape[0] <= 0 or query.shape[1] <= 0 or query.shape[2] <= 0:
@@ -153,21 +219,11 @@ def _validate_attention(query, cache, block_tables, context_lens, layer, validat
         raise ValueError("context_lens must use int32 or int64")
     if block_tables.shape[1] <= 0:
         raise ValueError("block_tables must contain at least one logical block")
-    if validate_inputs:
-        if bool(torch.any(context_lens <= 0).item()):
-            raise ValueError("context lengths must be positive")
-        max_context = block_tables.shape[1] * layout.block_size
-        if bool(torch.any(context_lens > max_context).item()):
-            raise ValueError("context length exceeds block table capacity")
-        if bool(torch.any(block_tables < 0).item()) or bool(
-            torch.any(block_tables >= layout.num_blocks).item()
-        ):
-            raise ValueError("block table contains an invalid physical block id")
-        if max_context_len and bool(torch.any(context_lens > max_context_len).item()):
-            raise ValueError("context length exceeds max_context_len")
+    check = _MetadataCheck(block_tables, context_lens, layout, max_context_len) if validate_inputs else _NoCheck()
     if query.dtype not in _DTYPES:
-        raise ValueError("query dtype must be float16, bfloat16 or float32")
-    return block_tables, context_lens
+        with check:
+            raise ValueError("query dtype must be float16, bfloat16 or float32")
+    return block_tables, context_lens, check
 
 
 def _aligned_rows(t: torch.Tensor) -> bool:
@@ -246,6 +302,7 @@ def _launch_attention(
     max_context_len: int | None,
     path: int = -1,
     events=None,
+    check=None,
 ) -> torch.Tensor:
     lib = _require_backend()
     if not _aligned_rows(query):
@@ -277,7 +334,9 @@ def _launch_attention(
     if events is not None:
         for i, ev in enumerate(events):
             args.events[i] = ev
-    with torch.cuda.device(query.device):
+    if check is not None:
+        check.wait()
+    with _on_device(query.device):
         stream = torch.cuda.current_stream(query.device).cuda_stream
         status = lib.ikl_paged_attention(ctypes.byref(args), ctypes.c_void_p(stream))
     _lib.check(status, "paged attention")
@@ -381,21 +440,23 @@ def paged_decode_attention_hip(
     recorded before the attention kernel, after it and after the split
     reduce, for timing).
     """
-    block_tables, context_lens = _validate_attention(
+    block_tables, context_lens, check = _validate_attention(
         query, cache, block_tables, context_lens, layer, validate_inputs, max_context_len
     )
-    return _launch_attention(
-        query,
-        cache,
-        block_tables,
-        context_lens,
-        scale,
-        layer,
-        query_group_size=0,
-        partition_size=partition_size,
-        max_context_len=max_context_len,
-        events=events,
-    )
+    with check:
+        return _launch_attention(
+            query,
+            cache,
+            block_tables,
+            context_lens,
+            scale,
+            layer,
+            query_group_size=0,
+            partition_size=partition_size,
+            max_context_len=max_context_len,
+            events=events,
+            check=check,
+        )
 
 
 def paged_decode_attention_hip_grouped(
@@ -422,35 +483,37 @@ def paged_decode_attention_hip_grouped(
     whatever the group size: a smaller group would only read K/V once more
     per group (MQA 32/1, batch 64: 66.7 µs with groups of 8 against 35.5 µs).
     """
-    block_tables, context_lens = _validate_attention(
+    block_tables, context_lens, check = _validate_attention(
         query, cache, block_tables, context_lens, layer, validate_inputs, max_context_len
     )
-    if query_group_size not in (1, 2, 4, 8):
-        raise ValueError("query_group_size must be one of 1, 2, 4, or 8")
-    heads_per_kv = query.shape[1] // cache.layout.num_kv_heads
-    path_name = paged_decode_grouped_path(
-        dtype=query.dtype,
-        head_dim=cache.layout.head_dim,
-        table_width=block_tables.shape[1],
-        heads_per_kv=heads_per_kv,
-        query_group_size=query_group_size,
-        block_size=cache.layout.block_size,
-    )
-    return _launch_attention(
-        query,
-        cache,
-        block_tables,
-        context_lens,
-        scale,
-        layer,
-        query_group_size=1 if heads_per_kv == 1 else (0 if path_name == "mfma_grouped" else query_group_size),
-        partition_size=partition_size,
-        max_context_len=max_context_len,
-        # the FP8 cache is read by the MFMA family only, and partition_size -2
-        # (the balanced split) leaves the family to the library, which runs
-        # it on the MFMA family (MHA included) where that supports the shape
-        path=-1 if cache.fp8 or partition_size == -2 else _PATH_IDS[path_name],
-    )
+    with check:
+        if query_group_size not in (1, 2, 4, 8):
+            raise ValueError("query_group_size must be one of 1, 2, 4, or 8")
+        heads_per_kv = query.shape[1] // cache.layout.num_kv_heads
+        path_name = paged_decode_grouped_path(
+            dtype=query.dtype,
+            head_dim=cache.layout.head_dim,
+            table_width=block_tables.shape[1],
+            heads_per_kv=heads_per_kv,
+            query_group_size=query_group_size,
+            block_size=cache.layout.block_size,
+        )
+        return _launch_attention(
+            query,
+            cache,
+            block_tables,
+            context_lens,
+            scale,
+            layer,
+            query_group_size=1 if heads_per_kv == 1 else (0 if path_name == "mfma_grouped" else query_group_size),
+            partition_size=partition_size,
+            max_context_len=max_context_len,
+            check=check,
+            # the FP8 cache is read by the MFMA family only, and partition_size -2
+            # (the balanced split) leaves the family to the library, which runs
+            # it on the MFMA family (MHA included) where that supports the shape
+            path=-1 if cache.fp8 or partition_size == -2 else _PATH_IDS[path_name],
+        )
 
 
 def append_kv_hip(key: torch.Tensor, value: torch.Tensor, cache, slots: torch.Tensor, layer: int = 0) -> None:
@@ -611,9 +674,10 @@ class PreparedPagedAttention:
                  query_group_size: int = 0, partition_size: int | None = None,
                  max_context_len: int | None = None, validate_inputs: bool = True):
         self._lib = _require_backend()
-        block_tables, context_lens = _validate_attention(
+        block_tables, context_lens, check = _validate_attention(
             query, cache, block_tables, context_lens, layer, validate_inputs, max_context_len
         )
+        check.wait()
         if not _aligned_rows(query):
             raise ValueError("query rows must be 16-byte aligned for a prepared launch")
         for tensor in (cache.k, cache.v):
