@@ -319,6 +319,54 @@ int32_t ikl_check_metadata(const void *tables, int32_t table_type, int64_t table
  * code when the launch failed. */
 int32_t ikl_check_metadata_wait(const uint32_t *flags, int32_t count, void *stream);
 
+/* RMSNorm of x [rows, cols] (row strides in elements, rows 16-byte aligned),
+ * after an optional residual add: sum = x + delta (rounded to the dtype; sum
+ * may be x), out = weight * round((sum or x) * rsqrt(mean(.^2) + eps)), each
+ * product rounded once (the norm of hf_benchmark.py:408-454's model). */
+typedef struct ikl_norm_args {
+  const void *x;
+  const void *delta;  /* NULL: no residual add */
+  const void *weight; /* [cols] */
+  void *sum;          /* with delta */
+  void *out;
+  int64_t x_stride, delta_stride, sum_stride, out_stride;
+  int64_t rows, cols;
+  int32_t dtype; /* enum ikl_dtype: F16, BF16, F32 */
+  float eps;
+  int32_t packed; /* 1: out in operand order (16 * cols elements, 16-bit, rows <= 16, cols a multiple of 64) */
+} ikl_norm_args;
+int ikl_add_rms_norm(const ikl_norm_args *args, void *stream);
+
+/* out = round(silu(gate)) * up over `count` contiguous elements. */
+int ikl_silu_mul(const void *gate, const void *up, void *out, int64_t count, int32_t dtype, void *stream);
+
+/* Linear layers over the few rows of a decode step, fp16 / bf16:
+ * y[i] = x weight[i]^T for up to three weights [out_cols, cols] (contiguous)
+ * that share x [rows, cols]. In operand order, 8-column piece c of row r of a
+ * 16-row matrix is piece (c / 4) * 64 + (c % 4) * 16 + r of the buffer; rows
+ * past `rows` may hold anything.
+ * epilogue 1: y[0] = residual + round(x weight[0]^T) (y[0] may be residual);
+ * epilogue 2: y[0] = round(silu(round(x weight[0]^T))) * round(x weight[1]^T). */
+#define IKL_DECODE_LINEAR_MAX_ROWS 16
+typedef struct ikl_decode_linear_args {
+  const void *x;
+  int64_t x_stride;
+  const void *weight[3];
+  void *y[3];
+  int64_t y_stride[3];
+  int64_t out_cols[3];
+  const void *residual;
+  int64_t residual_stride;
+  int64_t cols;
+  int32_t rows;
+  int32_t num_weights;
+  int32_t epilogue; /* 0 none, 1 residual, 2 silu(gate) * up */
+  int32_t dtype;
+  int32_t x_packed; /* 1: x in operand order (x_stride unused) */
+  int32_t y_packed; /* 1: y[0] of epilogue 2 in operand order */
+} ikl_decode_linear_args;
+int ikl_decode_linear(const ikl_decode_linear_args *args, void *stream);
+
 /* KV append (in place). Slots outside [0, num_blocks*block_size) are skipped,
  * never written. Replaces append.py:69-106 / cache.py:156-189. */
 int ikl_append_kv(const ikl_append_args *args, void *stream);

@@ -32,6 +32,9 @@ EXPORTED_SYMBOLS = (
     "ikl_last_error",
     "ikl_version",
     "ikl_abi_version",
+    "ikl_add_rms_norm",
+    "ikl_silu_mul",
+    "ikl_decode_linear",
     "ikl_check_metadata",
     "ikl_check_metadata_wait",
     "ikl_append_kv",
@@ -243,6 +246,51 @@ class LaunchConfig(ctypes.Structure):
     ]
 
 
+class NormArgs(ctypes.Structure):
+    """Mirror of ikl_norm_args."""
+
+    _fields_ = [
+        ("x", _c_ptr),
+        ("delta", _c_ptr),
+        ("weight", _c_ptr),
+        ("sum", _c_ptr),
+        ("out", _c_ptr),
+        ("x_stride", _c_i64),
+        ("delta_stride", _c_i64),
+        ("sum_stride", _c_i64),
+        ("out_stride", _c_i64),
+        ("rows", _c_i64),
+        ("cols", _c_i64),
+        ("dtype", _c_i32),
+        ("eps", ctypes.c_float),
+        ("packed", _c_i32),
+    ]
+
+
+class DecodeLinearArgs(ctypes.Structure):
+    """Mirror of ikl_decode_linear_args."""
+
+    _fields_ = [
+        ("x", _c_ptr),
+        ("x_stride", _c_i64),
+        ("weight", _c_ptr * 3),
+        ("y", _c_ptr * 3),
+        ("y_stride", _c_i64 * 3),
+        ("out_cols", _c_i64 * 3),
+        ("residual", _c_ptr),
+        ("residual_stride", _c_i64),
+        ("cols", _c_i64),
+        ("rows", _c_i32),
+        ("num_weights", _c_i32),
+        ("epilogue", _c_i32),
+        ("dtype", _c_i32),
+        ("x_packed", _c_i32),
+        ("y_packed", _c_i32),
+    ]
+
+
+DECODE_LINEAR_MAX_ROWS = 16  # IKL_DECODE_LINEAR_MAX_ROWS
+
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 _load_error: str | None = None
@@ -255,6 +303,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ikl_version.argtypes = []
     lib.ikl_abi_version.restype = _c_i32
     lib.ikl_abi_version.argtypes = []
+    lib.ikl_add_rms_norm.restype = ctypes.c_int
+    lib.ikl_add_rms_norm.argtypes = [ctypes.POINTER(NormArgs), _c_ptr]
+    lib.ikl_silu_mul.restype = ctypes.c_int
+    lib.ikl_silu_mul.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i32, _c_ptr]
+    lib.ikl_decode_linear.restype = ctypes.c_int
+    lib.ikl_decode_linear.argtypes = [ctypes.POINTER(DecodeLinearArgs), _c_ptr]
     lib.ikl_check_metadata.restype = _c_i32
     lib.ikl_check_metadata.argtypes = [_c_ptr, _c_i32, _c_i64, _c_i64, _c_ptr, _c_i32, _c_i64, _c_i64, _c_i64,
                                        _c_i64, _c_i64, _c_i64, _c_ptr, _c_i32, _c_ptr]

@@ -25,6 +25,7 @@ SOURCES = (
     "abi.hip",
     "append_kv.hip",
     "check_metadata.hip",
+    "layer_ops.hip",
     "paged_decode.hip",
     "paged_decode_mfma.hip",
     "paged_prefill.hip",

@@ -29,7 +29,7 @@ from typing import Any, Sequence
 import torch
 from torch import nn
 
-from . import ops
+from . import layer_ops, ops
 from .cache import PagedKVCache
 from .decode import ATTENTION_BACKENDS, APPEND_BACKENDS, DecodeMetadata, percentile
 from .runtime import InferenceRuntime
@@ -307,9 +307,42 @@ class LlamaPagedDecodeRunner:
         else:
             ops.append_kv_hip(key.contiguous(), value.contiguous(), self.cache, slots, layer=layer)
 
-    def _mlp_residual(self, layer, hidden: torch.Tensor) -> torch.Tensor:
-        x = layer.post_attention_layernorm(hidden)
-        return hidden + layer.mlp.down_proj(layer.mlp.act_fn(layer.mlp.gate_proj(x)) * layer.mlp.up_proj(x))
+    def _add_norm(self, norm, hidden: torch.Tensor, delta: torch.Tensor | None, *, packed: bool = False):
+        """(hidden + delta, norm of it): one kernel for a plain RMSNorm.
+        `packed`: (norm, rows) for decode_linear, the norm in operand order
+        (rows set) where the kernel runs."""
+        if (layer_ops.plain_module(norm, RMSNorm) and layer_ops.kernels_apply(hidden)
+                and (delta is None or (type(delta) is torch.Tensor and delta.dtype == hidden.dtype
+                                       and delta.shape == hidden.shape and delta.device == hidden.device))
+                and layer_ops.norm_fits(norm.weight, hidden)):
+            hidden, x = layer_ops.add_rms_norm(hidden, delta, norm.weight, norm.variance_epsilon, packed=packed)
+            return hidden, (x, hidden.shape[0]) if packed else x
+        if delta is not None:
+            hidden = hidden + delta
+        x = norm(hidden)
+        return hidden, (x, None) if packed else x
+
+    def _mlp(self, mlp, x: torch.Tensor) -> torch.Tensor:
+        gate, up = mlp.gate_proj(x), mlp.up_proj(x)
+        if (layer_ops.plain_module(mlp.act_fn, nn.SiLU) and not mlp.act_fn.inplace and layer_ops.kernels_apply(gate)
+                and layer_ops.silu_mul_fits(gate, up)):
+            return mlp.down_proj(layer_ops.silu_mul(gate, up))
+        return mlp.down_proj(mlp.act_fn(gate) * up)
+
+    def _decode_linears(self, layer, hidden: torch.Tensor) -> bool:
+        """Whether the decode linear kernels restate this layer's linears and
+        activation on `hidden`: the q/k/v projections, the o projection and
+        its residual add, the gated MLP and its."""
+        att, mlp = layer.self_attn, layer.mlp
+        return (layer_ops.kernels_apply(hidden)
+                and all(layer_ops.linear_fits(p, hidden)
+                        for p in (att.q_proj, att.k_proj, att.v_proj, mlp.gate_proj, mlp.up_proj))
+                and layer_ops.plain_module(mlp.act_fn, nn.SiLU) and not mlp.act_fn.inplace
+                and all(layer_ops.linear_weight_fits(p, hidden) and p.weight.shape[0] == hidden.shape[1]
+                        for p in (att.o_proj, mlp.down_proj))
+                and att.q_proj.weight.shape[0] == att.o_proj.weight.shape[1]
+                and mlp.gate_proj.weight.shape == mlp.up_proj.weight.shape
+                and mlp.gate_proj.weight.shape[0] == mlp.down_proj.weight.shape[1])
 
     # ------------------------------------------------------- decode forward
     def _forward_decode(self, token_ids: torch.Tensor, requests, positions) -> torch.Tensor:
@@ -331,12 +364,20 @@ class LlamaPagedDecodeRunner:
         fused = self.append_backend != "torch"
         if fused:
             cos2, sin2 = cos.reshape(n, self.head_dim).contiguous(), sin.reshape(n, self.head_dim).contiguous()
+        delta = None  # the last block's output, not yet added to `hidden`
         for li, layer in enumerate(m.layers):
-            x = layer.input_layernorm(hidden)
             att = layer.self_attn
-            q = att.q_proj(x).view(n, self.num_heads, self.head_dim)
-            k = att.k_proj(x).view(n, self.num_kv_heads, self.head_dim)
-            v = att.v_proj(x).view(n, self.num_kv_heads, self.head_dim)
+            kernels = self._decode_linears(layer, hidden)
+            hidden, x = self._add_norm(layer.input_layernorm, hidden, delta, packed=kernels)
+            delta = None
+            if kernels:
+                q, k, v = layer_ops.decode_linear(x[0], (att.q_proj.weight, att.k_proj.weight, att.v_proj.weight),
+                                                  rows=x[1])
+            else:
+                q, k, v = att.q_proj(x), att.k_proj(x), att.v_proj(x)
+            q = q.view(n, self.num_heads, self.head_dim)
+            k = k.view(n, self.num_kv_heads, self.head_dim)
+            v = v.view(n, self.num_kv_heads, self.head_dim)
             if fused:  # RoPE of q and k + append of rope(k), v: one launch (q rotated in place)
                 ops.rope_append_kv_hip(q, k, v, cos2, sin2, self.cache, slots, layer=li)
             else:
@@ -344,9 +385,17 @@ class LlamaPagedDecodeRunner:
                 self._append(li, slots, k, v)
             o = self._attend(q.contiguous(), self.cache, tables, lens, layer=li, validate_inputs=validate and li == 0,
                              max_context_len=self._max_ctx)
-            hidden = hidden + att.o_proj(o.reshape(n, self.num_heads * self.head_dim))
-            hidden = self._mlp_residual(layer, hidden)
-        return self.model.lm_head(m.norm(hidden))
+            o = o.reshape(n, self.num_heads * self.head_dim)
+            if kernels:
+                hidden = layer_ops.decode_linear(o, (att.o_proj.weight,), residual=hidden)
+                _, x = self._add_norm(layer.post_attention_layernorm, hidden, None, packed=True)
+                x = layer_ops.decode_linear(x[0], (layer.mlp.gate_proj.weight, layer.mlp.up_proj.weight), rows=x[1],
+                                            silu=True, packed=True)
+                hidden = layer_ops.decode_linear(x, (layer.mlp.down_proj.weight,), rows=n, residual=hidden)
+            else:
+                hidden, x = self._add_norm(layer.post_attention_layernorm, hidden, att.o_proj(o))
+                delta = self._mlp(layer.mlp, x)
+        return self.model.lm_head(self._add_norm(m.norm, hidden, delta)[1])
 
     # ------------------------------------------------------ prefill forward
     def _prefix_attention(self, q: torch.Tensor, layer: int, tables: torch.Tensor, starts, ends) -> torch.Tensor:
@@ -411,8 +460,9 @@ class LlamaPagedDecodeRunner:
         if self.prefill_attention == "hip":
             prefill = ops.PreparedPagedPrefill(self.cache, tables, list(starts), list(ends),
                                                num_heads=self.num_heads, query_width=t)
+        delta = None  # the last block's output, not yet added to `hidden`
         for li, layer in enumerate(m.layers):
-            x = layer.input_layernorm(hidden)
+            hidden, x = self._add_norm(layer.input_layernorm, hidden, delta)
             att = layer.self_attn
             q = att.q_proj(x).view(b, t, self.num_heads, self.head_dim)
             k = att.k_proj(x).view(b, t, self.num_kv_heads, self.head_dim)
@@ -431,9 +481,10 @@ class LlamaPagedDecodeRunner:
                 prefill(q.transpose(1, 2), li, out=o.transpose(1, 2))
             else:
                 o = self._prefix_attention(q, li, tables, starts, ends)
-            hidden = hidden + att.o_proj(o.reshape(b, t, self.num_heads * self.head_dim))
-            hidden = self._mlp_residual(layer, hidden)
-        return self.model.lm_head(m.norm(hidden))
+            hidden, x = self._add_norm(layer.post_attention_layernorm, hidden,
+                                       att.o_proj(o.reshape(b, t, self.num_heads * self.head_dim)))
+            delta = self._mlp(layer.mlp, x)
+        return self.model.lm_head(self._add_norm(m.norm, hidden, delta)[1])
 
     # -------------------------------------------------------------- hooks
     def _prefill(self, request: InferenceRequest, start: int, end: int) -> None:

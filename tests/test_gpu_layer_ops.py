@@ -1,0 +1,128 @@
+"""The Llama layer kernels against the modules they restate, computed in
+float64 from the same 16-bit inputs with the modules' roundings: RMSNorm
+(+ residual) over row widths at the edges of a workgroup's pieces, SiLU * up,
+and the decode linears over row counts at the edges of their 16-row tiles,
+contraction lengths at the edges of a wave's steps, and one to three weights
+with each epilogue. A result may land on the other side of a rounding
+boundary: the bound is one ulp of the dtype per rounding of the sequence."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ULP = {torch.bfloat16: 2.0**-7, torch.float16: 2.0**-10, torch.float32: 2.0**-21}
+
+
+def _close(got, expected, dtype, roundings, floor):
+    err = (got.double() - expected).abs()
+    bound = roundings * ULP[dtype] * (expected.abs() + floor)
+    assert bool((err <= bound).all()), (float((err - bound).max()), float(err.max()))
+
+
+def _norm(x, w, eps):
+    d = x.double()
+    d = (d * torch.rsqrt(d.square().mean(-1, keepdim=True) + eps)).to(x.dtype)
+    return w.double() * d.double()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 24), (16, 2048), (5, 2056), (17, 4096)])
+@pytest.mark.parametrize("add", [False, True])
+def test_add_rms_norm(dtype, rows, cols, add):
+    from inferkernellab_amd import layer_ops as lo
+
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = torch.randn(rows, cols, device="cuda", generator=g).to(dtype)
+    wide = torch.randn(rows, 2 * cols, device="cuda", generator=g).to(dtype)
+    delta = wide[:, :cols] if add else None  # strided rows
+    w = (1 + 0.1 * torch.randn(cols, device="cuda", generator=g)).to(dtype)
+    with torch.no_grad():
+        assert lo.norm_fits(w, x)
+        total, out = lo.add_rms_norm(x, delta, w, 1e-6)
+    expected = x + delta if add else x
+    assert torch.equal(total, expected)
+    _close(out, _norm(expected, w, 1e-6), dtype, 2, 1e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(8,), (3, 40), (257, 512)])
+def test_silu_mul(dtype, shape):
+    from inferkernellab_amd import layer_ops as lo
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    gate, up = (4 * torch.randn(2, *shape, device="cuda", generator=g)).to(dtype)
+    gate.view(-1)[:4] = torch.tensor([float("-inf"), 100.0, -100.0, 0.0], device="cuda")
+    up.view(-1)[0] = 1.0
+    assert lo.silu_mul_fits(gate, up)
+    got = lo.silu_mul(gate, up)
+    d = gate.double()
+    expected = (d / (1 + torch.exp(-d))).to(dtype).double() * up.double()
+    assert bool(torch.isnan(got.view(-1)[0])) and bool(torch.isnan(expected.view(-1)[0]))  # -inf * 0
+    _close(got.view(-1)[1:], expected.view(-1)[1:], dtype, 2, 1e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 7, 15, 16])
+@pytest.mark.parametrize("cols,outs", [(64, (16,)), (512, (48, 16, 32)), (576, (64, 16)), (2048, (256, 64, 64)),
+                                       (2112, (32,)), (5632, (16,))])
+def test_decode_linear(dtype, rows, cols, outs):
+    from inferkernellab_amd import layer_ops as lo
+
+    g = torch.Generator(device="cuda").manual_seed(rows + cols + len(outs))
+    x = torch.randn(rows, 2 * cols, device="cuda", generator=g).to(dtype)[:, cols:]  # strided rows
+    ws = [(torch.randn(n, cols, device="cuda", generator=g) * cols**-0.5).to(dtype) for n in outs]
+    products = [x.double() @ w.double().t() for w in ws]  # of magnitude about 1
+    got = lo.decode_linear(x, ws)
+    for y, e in zip([got] if len(ws) == 1 else got, products):
+        _close(y, e, dtype, 1, 0.25)
+    res = torch.randn(rows, outs[0], device="cuda", generator=g).to(dtype)
+    y = lo.decode_linear(x, ws[:1], residual=res)
+    _close(y, res.double() + products[0].to(dtype).double(), dtype, 2, 0.5)
+    up = torch.flip(ws[0], (0,)).contiguous()
+    y = lo.decode_linear(x, [ws[0], up], silu=True)
+    a, b = products[0].to(dtype).double(), torch.flip(products[0], (1,)).to(dtype).double()
+    s = (a / (1 + torch.exp(-a))).to(dtype).double()
+    _close(y, s * b, dtype, 4, 1.0)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 16])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_operand_order_changes_no_value(dtype, rows):
+    """norm -> gate * up -> down with the tensors between them in operand
+    order, against the same kernels over plain rows: bit for bit."""
+    from inferkernellab_amd import layer_ops as lo
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, 576, device="cuda", generator=g).to(dtype)
+    w = torch.randn(576, device="cuda", generator=g).to(dtype)
+    gate, up = (0.05 * torch.randn(2, 704, 576, device="cuda", generator=g)).to(dtype)
+    down = (0.05 * torch.randn(576, 704, device="cuda", generator=g)).to(dtype)
+    _, a = lo.add_rms_norm(x, None, w, 1e-6)
+    b = lo.decode_linear(a, (gate, up), silu=True)
+    c = lo.decode_linear(b, (down,), residual=x)
+    _, pa = lo.add_rms_norm(x, None, w, 1e-6, packed=True)
+    pb = lo.decode_linear(pa, (gate, up), rows=rows, silu=True, packed=True)
+    assert torch.equal(lo.decode_linear(pb, (down,), rows=rows, residual=x), c)
+    assert torch.equal(lo.decode_linear(pa, (gate,), rows=rows), lo.decode_linear(a, (gate,)))
+
+
+def test_what_the_kernels_do_not_restate_is_left_to_the_module():
+    from inferkernellab_amd import layer_ops as lo
+
+    x = torch.zeros(4, 128, dtype=torch.bfloat16, device="cuda")
+    lin = torch.nn.Linear(128, 32, bias=False, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        assert lo.kernels_apply(x) and lo.linear_fits(lin, x)
+        assert not lo.linear_fits(lin, torch.zeros(17, 128, dtype=torch.bfloat16, device="cuda"))
+        assert not lo.linear_fits(lin, x.float()) and not lo.linear_fits(lin, x[:0])
+        assert not lo.linear_fits(torch.nn.Linear(128, 24, bias=False, device="cuda", dtype=torch.bfloat16), x)
+        assert not lo.linear_fits(torch.nn.Linear(128, 32, device="cuda", dtype=torch.bfloat16), x)
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert not lo.kernels_apply(x)
+        handle = lin.register_forward_hook(lambda *a: None)
+        assert not lo.linear_fits(lin, x)
+        handle.remove()
+        torch.nn.utils.parametrizations.weight_norm(lin)
+        assert not lo.linear_fits(lin, x)
+    assert not lo.kernels_apply(x)  # autograd may record
