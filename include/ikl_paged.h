@@ -267,6 +267,12 @@ typedef struct ikl_paged_prefill_args {
  * read outside the cache. Replaces attention.py:230-321. */
 int ikl_paged_prefill_attention(const ikl_paged_prefill_args *args, void *stream);
 
+/* How a matrix-core prefill launch splits its keys: 1, 2 or 4 waves share
+ * each row (launches that leave the chip idle), 0 when all waves of a
+ * workgroup walk the keys together, or on the other family. Planning only:
+ * tensors are not looked at. Negative on invalid sizes. */
+int32_t ikl_paged_prefill_key_groups(const ikl_paged_prefill_args *args);
+
 /* Kernel family a prefill launch uses: IKL_PATH_MFMA_GROUPED for fp16/bf16
  * with head_dim in {32, 64, 96, 128} and block_size a multiple of 16, else
  * IKL_PATH_SCALAR_GROUPED. dtype: enum ikl_dtype. */

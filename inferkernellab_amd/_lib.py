@@ -46,6 +46,7 @@ EXPORTED_SYMBOLS = (
     "ikl_rope_append_kv",
     "ikl_paged_prefill_attention",
     "ikl_paged_prefill_path",
+    "ikl_paged_prefill_key_groups",
     "ikl_paged_decode_step",
     "ikl_paged_decode_step_fused",
     "ikl_paged_decode_step_workspace_size",
@@ -328,6 +329,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ikl_rope_append_kv.argtypes = [ctypes.POINTER(RopeAppendArgs), _c_ptr]
     lib.ikl_paged_prefill_attention.restype = ctypes.c_int
     lib.ikl_paged_prefill_attention.argtypes = [ctypes.POINTER(PagedPrefillArgs), _c_ptr]
+    lib.ikl_paged_prefill_key_groups.restype = _c_i32
+    lib.ikl_paged_prefill_key_groups.argtypes = [ctypes.POINTER(PagedPrefillArgs)]
     lib.ikl_paged_prefill_path.restype = _c_i32
     lib.ikl_paged_prefill_path.argtypes = [_c_i32, _c_i32, _c_i32]
     lib.ikl_paged_attention_noalloc.restype = ctypes.c_int

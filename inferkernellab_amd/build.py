@@ -30,6 +30,7 @@ SOURCES = (
     "paged_decode_mfma.hip",
     "paged_prefill.hip",
     "paged_prefill_f32.hip",
+    "paged_prefill_split.hip",
     "rope_append.hip",
     "read_probe.hip",
 )
@@ -59,6 +60,7 @@ COMMON_FLAGS = [
 # 51.4 us at head_dim 64).
 SOURCE_FLAGS = {
     "paged_prefill.hip": ["-fno-honor-nans"],
+    "paged_prefill_split.hip": ["-fno-honor-nans"],
     "paged_prefill_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "paged_decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }

@@ -1,5 +1,6 @@
 // Parameters and block-table helpers shared by the paged prefill kernels
 // (paged_prefill.hip: 16-bit matrix cores and the wide-row fallback;
+// paged_prefill_split.hip: 16-bit matrix cores, keys split between waves;
 // paged_prefill_f32.hip: fp32 matrix cores).
 #pragma once
 
@@ -29,6 +30,7 @@ struct PrefillParams {
   int64_t row_blocks;  // workgroups per (request, kv head) of the MFMA kernel
   int64_t bh_pad;      // batch * num_kv_heads rounded up to a multiple of 8
   int32_t stream_major;  // each XCD takes its (request, kv head) prefixes one after another
+  int32_t paired;        // one resident round: the shortest row blocks share CUs with the longest
   int32_t num_heads;
   int32_t num_kv_heads;
   int32_t heads_per_kv;
@@ -51,6 +53,11 @@ struct PrefillParams {
 // set here.
 constexpr int PREFILL_F32_MAX_DIM = 256;
 hipError_t launch_prefill_f32(PrefillParams p, int dtype, hipStream_t s);
+
+// Launches paged_prefill_split_kernel (what the 16-bit kernel takes) with
+// `groups` (2 or 4) waves on every row; p.row_blocks and p.bh_pad are set
+// here.
+hipError_t launch_prefill_split(PrefillParams p, int dtype, int groups, hipStream_t s);
 
 namespace {
 
@@ -80,6 +87,20 @@ __device__ inline void pf_range(const PrefillParams &p, int64_t b, int64_t *star
 
 __device__ inline int64_t pf_logical(const PrefillParams &p, int64_t pos) {
   return p.bs_shift >= 0 ? (pos >> p.bs_shift) : pos / p.block_size;
+}
+
+// Two E4M3 codes times one fp32 scale -> two 16-bit values (one rounding).
+template <typename Tag>
+__device__ inline uint32_t fp8x2_scaled(uint32_t w, float scale, bool hi);
+template <>
+__device__ inline uint32_t fp8x2_scaled<bf16_tag>(uint32_t w, float scale, bool hi) {
+  return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, true)
+                                        : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, false));
+}
+template <>
+__device__ inline uint32_t fp8x2_scaled<f16_tag>(uint32_t w, float scale, bool hi) {
+  return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, true)
+                                        : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, false));
 }
 
 }  // namespace

@@ -10,7 +10,9 @@
 // Two kernel families:
 //
 //  * MFMA (fp16 / bf16, head_dim 32k <= 128, block_size % 16 == 0):
-//    paged_prefill_mfma_kernel. A workgroup of 4 waves takes 64 * NG query
+//    launches that fill the chip run paged_prefill_mfma_kernel, smaller ones
+//    paged_prefill_split_kernel (paged_prefill_split.hip; the rule is
+//    prefill_key_groups). A workgroup of 4 waves takes 64 * NG query
 //    rows of one (request, kv head) — a row is one (token, query head) pair,
 //    token-major, so the heads sharing a KV head sit in consecutive rows —
 //    and streams the request's keys in 32-token tiles that the workgroup
@@ -54,20 +56,6 @@ constexpr int PWAVES = 4;  // waves per workgroup
 constexpr int PREFILL_NG = 2;
 constexpr int PF = 2;  // tiles held in registers ahead of the one being staged
 #define IKL_PREFILL_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(2, 8)))
-
-// Two E4M3 codes times one fp32 scale -> two 16-bit values (one rounding).
-template <typename Tag>
-__device__ inline uint32_t fp8x2_scaled(uint32_t w, float scale, bool hi);
-template <>
-__device__ inline uint32_t fp8x2_scaled<bf16_tag>(uint32_t w, float scale, bool hi) {
-  return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, true)
-                                        : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, false));
-}
-template <>
-__device__ inline uint32_t fp8x2_scaled<f16_tag>(uint32_t w, float scale, bool hi) {
-  return __builtin_bit_cast(uint32_t, hi ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, true)
-                                        : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, false));
-}
 
 // KV8: the cache holds E4M3 codes with per-row scales. The copy waves load
 // the codes (half the bytes) and each row's scale, and stage
@@ -582,10 +570,13 @@ __global__ __launch_bounds__(64) void paged_prefill_scalar_kernel(const PrefillP
 
 template <typename Tag, int NG, bool KV8>
 hipError_t launch_mfma_dim(int d, const PrefillParams &p, dim3 grid, hipStream_t s) {
+  // 32 dims, and 96 over the FP8 cache, run the split kernel at every size
   switch (d) {
-    case 32: paged_prefill_mfma_kernel<Tag, 32, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
     case 64: paged_prefill_mfma_kernel<Tag, 64, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
-    case 96: paged_prefill_mfma_kernel<Tag, 96, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
+    case 96:
+      if constexpr (!KV8) paged_prefill_mfma_kernel<Tag, 96, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p);
+      else return hipErrorInvalidValue;
+      break;
     default: paged_prefill_mfma_kernel<Tag, 128, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
   }
   return hipGetLastError();
@@ -597,6 +588,34 @@ bool prefill_mfma_supported(int dtype, int head_dim, int block_size) {
          block_size % 16 == 0;
 }
 
+// Waves per row of the split kernel (paged_prefill_split.hip) a launch of the
+// 16-bit matrix cores runs with, or 0 for paged_prefill_mfma_kernel. `blocks`:
+// 128-row workgroups (two are resident per CU, 512 on the chip's 256 CUs).
+// Measured on 32/8 heads, us for 0 / 1 / 2 / 4 (bf16, 128 dims unless said):
+//   a quarter of the CUs: 4 x (2000 + 64 tokens)  57.6 / 51.9 / 36.5 / 28.9
+//   the CUs once:  1 x 1024                       32.1 / 29.3 / 23.8 / 49.7
+//                  8 x (2000 + 128), FP8 cache    64.2 / 58.0 / 54.9 / 123
+//   one resident round: 2 x 1024                  36.6 / 32.8 / 38.3 / -
+// Two rounds gain where the rows sit behind long prefixes (equal, long
+// chains; a table of at least twice the query width stands for that):
+//   4 x (2048 + 517-1024 tokens) 150.7 / 144.8, FP8 cache 166.3 / 152.9,
+//   64 dims 104.0 / 93.9; but 6 x 512 from position 0: 30.5 / 34.4.
+// Beyond that a launch runs at the chip's power limit, where the 16x16x32
+// MFMA is 2-5 % ahead, except for 32 dims (4 x 2048: 78.4 / 66.2) and 96 dims
+// over the FP8 cache (8 x 4096: 1170 / 1091).
+int prefill_key_groups(int64_t blocks, int64_t cap_tokens, int64_t width, int head_dim, bool kv8) {
+  if (blocks <= 64) return 4;
+  if (blocks <= 256) return 2;
+  if (blocks <= 512 || (blocks <= 1024 && cap_tokens >= 2 * width)) return 1;
+  return head_dim == 32 || (head_dim == 96 && kv8) ? 1 : 0;
+}
+
+int64_t prefill_blocks(const ikl_paged_prefill_args *a) {
+  const int64_t rows = a->query_width * (a->num_heads / a->num_kv_heads);
+  constexpr int64_t rows_per_wg = 16 * PREFILL_NG * PWAVES;  // RWG of the kernel
+  return (rows + rows_per_wg - 1) / rows_per_wg * ((a->batch * a->num_kv_heads + 7) / 8 * 8);
+}
+
 bool aligned(const void *ptr, int64_t bytes) { return ((uintptr_t)ptr) % bytes == 0; }
 
 }  // namespace
@@ -606,6 +625,14 @@ using namespace ikl;
 
 extern "C" int32_t ikl_paged_prefill_path(int32_t dtype, int32_t head_dim, int32_t block_size) {
   return prefill_mfma_supported(dtype, head_dim, block_size) ? IKL_PATH_MFMA_GROUPED : IKL_PATH_SCALAR_GROUPED;
+}
+
+extern "C" int32_t ikl_paged_prefill_key_groups(const ikl_paged_prefill_args *a) {
+  if (!a || a->batch <= 0 || a->query_width <= 0 || a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0)
+    return fail(IKL_EINVAL, "ikl_paged_prefill_key_groups: invalid arguments");
+  if (!prefill_mfma_supported(a->dtype, a->head_dim, a->block_size) || a->path == IKL_PATH_SCALAR_GROUPED) return 0;
+  return prefill_key_groups(prefill_blocks(a), a->table_width * a->block_size, a->query_width, a->head_dim,
+                            a->cache_dtype == IKL_FP8_E4M3);
 }
 
 extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void *stream) {
@@ -716,20 +743,21 @@ extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void
   hipError_t err;
   if (path == IKL_PATH_MFMA_GROUPED) {
     constexpr int NG = PREFILL_NG;
-    const int64_t rows = a->query_width * p.heads_per_kv;
-    constexpr int64_t rows_per_wg = 16 * NG * PWAVES;  // RWG of the kernel
-    p.row_blocks = (rows + rows_per_wg - 1) / rows_per_wg;
+    const int64_t blocks = prefill_blocks(a);
     p.bh_pad = (a->batch * a->num_kv_heads + 7) / 8 * 8;
+    p.row_blocks = blocks / p.bh_pad;
     // stream-major once a prefix has enough row blocks to fill an XCD's
     // resident workgroups (32 CUs x 2). GQA 32/8 hd128 bf16, 8 x 4096
     // prompts: FETCH_SIZE 3.50 -> 0.67 x the algorithmic bytes, kernel
     // 1252 -> 1238 us. Over the FP8 cache (half the K/V bytes per tile) it
     // measured 1.5 % slower (1270 -> 1289 us) and stays off.
     p.stream_major = p.row_blocks >= 64 && !p.kv_fp8;
-    const int64_t blocks = p.row_blocks * p.bh_pad;
     if (blocks > 0x7fffffffLL) return fail(IKL_EINVAL, "ikl_paged_prefill_attention: launch too large");
     const dim3 grid((unsigned)blocks);
-    if (a->dtype == IKL_BF16)
+    const int groups = prefill_key_groups(blocks, p.cap_tokens, p.width, p.head_dim, kv8);
+    if (groups > 0)
+      err = launch_prefill_split(p, a->dtype, groups, s);
+    else if (a->dtype == IKL_BF16)
       err = p.kv_fp8 ? launch_mfma_dim<bf16_tag, NG, true>(a->head_dim, p, grid, s)
                      : launch_mfma_dim<bf16_tag, NG, false>(a->head_dim, p, grid, s);
     else

@@ -936,10 +936,11 @@ class PreparedPagedPrefill:
         a.scale = float(scale if scale is not None else layout.head_dim**-0.5)
         a.path = _PATH_IDS[self.path]
         self._args = a
+        self.key_groups = self._lib.ikl_paged_prefill_key_groups(ctypes.byref(a))
 
     def kernel_name(self) -> str:
         if self.path == "mfma_grouped":
-            return "paged_prefill_mfma_kernel"
+            return "paged_prefill_split_kernel" if self.key_groups else "paged_prefill_mfma_kernel"
         return "paged_prefill_f32_kernel" if self.shape[-1] <= 256 else "paged_prefill_scalar_kernel"
 
     def __call__(self, query: torch.Tensor, layer: int = 0, *, out: torch.Tensor | None = None,
