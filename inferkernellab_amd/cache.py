@@ -167,9 +167,9 @@ class PagedKVCache:
     def release_request(self, block_table, request_id: int | None = None) -> None:
         self.allocator.free(block_table, owner=request_id)
 
-    def slot_mapping(self, block_table, start: int, length: int) -> torch.Tensor:
+    def slot_mapping(self, block_table, start: int, length: int, *, device=None) -> torch.Tensor:
         """Physical slots of logical positions ``[start, start + length)``
-        (cache.py:113-129), int64 on the cache device."""
+        (cache.py:113-129), int64 on the cache device (or on `device`)."""
         bs = self.layout.block_size
         if start < 0 or length < 0:
             raise ValueError("start and length must be non-negative")
@@ -183,8 +183,9 @@ class PagedKVCache:
             raise ValueError("block_table contains an invalid physical block id")
         if length and (start + length - 1) // bs >= len(block_table):
             raise ValueError("block_table is shorter than the requested range")
-        positions = torch.arange(start, start + length, dtype=torch.long, device=self.device)
-        table = torch.as_tensor(block_table, dtype=torch.long, device=self.device)
+        device = self.device if device is None else device
+        positions = torch.arange(start, start + length, dtype=torch.long, device=device)
+        table = torch.as_tensor(block_table, dtype=torch.long, device=device)
         return table[positions // bs] * bs + positions % bs
 
     def _check_kv(self, key: torch.Tensor, value: torch.Tensor) -> None:

@@ -25,29 +25,32 @@ MAX_ROWS = _lib.DECODE_LINEAR_MAX_ROWS
 MAX_WEIGHT = 1 << 24
 
 
-def plain_module(module, cls) -> bool:
-    """True when calling `module` runs cls.forward and nothing else."""
+def unhooked(module) -> bool:
+    """True when nothing but the module's class sees a call of it."""
     return (
-        type(module) is cls
-        and not module._forward_hooks
+        not module._forward_hooks
         and not module._forward_pre_hooks
         and not module._backward_hooks
         and not module._backward_pre_hooks
         and "forward" not in module.__dict__
+        and not nn.modules.module._has_any_global_hook()
     )
+
+
+def plain_module(module, cls) -> bool:
+    """True when calling `module` runs cls.forward and nothing else."""
+    return type(module) is cls and unhooked(module)
 
 
 def kernels_apply(x: torch.Tensor) -> bool:
     """Whether a module call on `x` may be restated by a kernel at all: no
-    graph to record, no autocast, no hook on every module, a plain tensor on
-    a GPU."""
+    graph to record, no autocast, a plain tensor on a GPU."""
     return (
         type(x) is torch.Tensor
         and x.device.type == "cuda"
         and x.dtype in _DTYPES
         and not torch.is_grad_enabled()
         and not torch.is_autocast_enabled()
-        and not nn.modules.module._has_any_global_hook()
     )
 
 

@@ -151,6 +151,9 @@ def random_llama(config: LlamaConfig, *, seed: int = 0, device="cuda",
 
 
 # --------------------------------------------------------------- the runner
+CAPTURE_FREE = 4 << 30  # device memory that a step's capture is sure to fit in
+
+
 @dataclass
 class _StepBuffers:
     """Static device buffers of one captured decode step."""
@@ -163,6 +166,7 @@ class _StepBuffers:
     slots: torch.Tensor
     used: torch.Tensor | None = None
     graph: torch.cuda.CUDAGraph | None = None
+    staged: torch.Tensor | None = None  # pinned host copy of the step's fp32 logits
 
 
 @dataclass(frozen=True)
@@ -285,6 +289,7 @@ class LlamaPagedDecodeRunner:
         self._prompt_logits: dict[int, torch.Tensor] = {}
         self._next_logits: dict[int, torch.Tensor] = {}
         self._decode_logits: list[torch.Tensor] = []
+        self._staged: torch.Tensor | None = None
         self._padding = 0
         self._generated = {r.request_id: [] for r in self.requests}
         self._token_logprobs = {r.request_id: [] for r in self.requests}
@@ -430,7 +435,8 @@ class LlamaPagedDecodeRunner:
         return out.permute(0, 2, 1, 3).to(q.dtype)
 
     def _forward_prefill(self, token_ids: torch.Tensor, requests, starts, ends) -> torch.Tensor:
-        """Logits [B, T, vocab] of prompt chunks token_ids [B, T] (padded).
+        """Logits [B, vocab] at the end of each prompt chunk of token_ids
+        [B, T] (padded).
 
         With the HIP backends (the default) each layer runs two kernels
         around its projections: the fused RoPE + append over the batch's
@@ -449,7 +455,7 @@ class LlamaPagedDecodeRunner:
         if fused:
             slot_rows = torch.full((b, t), -1, dtype=torch.int32)
             for i, (r, s_, n) in enumerate(zip(requests, starts, spans)):
-                slot_rows[i, :n] = torch.as_tensor(self.cache.slot_mapping(r.block_table, s_, n), dtype=torch.int32)
+                slot_rows[i, :n] = self.cache.slot_mapping(r.block_table, s_, n, device="cpu")
             slots = slot_rows.reshape(-1).to(self.device)
             cos2, sin2 = cos.reshape(b * t, self.head_dim).contiguous(), sin.reshape(b * t, self.head_dim).contiguous()
         else:
@@ -484,7 +490,15 @@ class LlamaPagedDecodeRunner:
             hidden, x = self._add_norm(layer.post_attention_layernorm, hidden,
                                        att.o_proj(o.reshape(b, t, self.num_heads * self.head_dim)))
             delta = self._mlp(layer.mlp, x)
-        return self.model.lm_head(self._add_norm(m.norm, hidden, delta)[1])
+        # Only the chunks' last rows are read. Where a module between them
+        # and the logits is hooked or not a plain one, it sees all rows.
+        last = torch.tensor([n - 1 for n in spans], device=self.device)
+        rows = torch.arange(b, device=self.device)
+        if layer_ops.unhooked(m.norm) and layer_ops.plain_module(self.model.lm_head, nn.Linear):
+            hidden = hidden[rows, last]
+            delta = None if delta is None else delta[rows, last]
+            return self.model.lm_head(self._add_norm(m.norm, hidden, delta)[1])
+        return self.model.lm_head(self._add_norm(m.norm, hidden, delta)[1])[rows, last]
 
     # -------------------------------------------------------------- hooks
     def _prefill(self, request: InferenceRequest, start: int, end: int) -> None:
@@ -500,10 +514,10 @@ class LlamaPagedDecodeRunner:
             ids[row, : e - s] = torch.tensor(self.prompts[r.request_id][s:e])
         self._padding += len(requests) * width - sum(spans)
         logits = self._forward_prefill(ids.to(self.device), requests, starts, ends)
-        for row, (r, e, n) in enumerate(zip(requests, ends, spans)):
+        for row, (r, e) in enumerate(zip(requests, ends)):
             if e == len(self.prompts[r.request_id]):
-                self._prompt_logits[r.request_id] = logits[row, n - 1].detach()
-                self._next_logits[r.request_id] = logits[row, n - 1].detach()
+                self._prompt_logits[r.request_id] = logits[row].detach()
+                self._next_logits[r.request_id] = logits[row].detach()
 
     def _sample(self, logits: torch.Tensor, gen: torch.Generator):
         """(token, policy log-prob, sampling log-prob) as hf_benchmark.py:578-606."""
@@ -548,22 +562,48 @@ class LlamaPagedDecodeRunner:
                 slots=torch.zeros(n, dtype=torch.int32, device=self.device),
             )
             st.used = torch.empty_like(st.logits)
+            st.staged = torch.empty(st.logits.shape, dtype=torch.float32, pin_memory=True)
             side = torch.cuda.Stream(self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
             with torch.cuda.stream(side):
                 self._graph_body(st)  # this step's execution
             torch.cuda.current_stream(self.device).wait_stream(side)
-            st.graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(st.graph):
-                self._graph_body(st)
+            st.graph = self._capture(st, side)
             self._graphs[key] = st
         else:
             st.graph.replay()
-        self._decode_logits.append(st.used.float().cpu())
+        # The previous step's logits leave their staging buffer while this
+        # step runs; this one's follow it into the buffer.
+        self._collect_logits()
+        st.staged.copy_(st.used, non_blocking=True)
+        self._staged = st.staged
         toks = st.tok.tolist()
         for i, r in enumerate(requests):
             self._generated[r.request_id].append(int(toks[i]))
             self._next_logits[r.request_id] = st.logits[i]
+
+    def _collect_logits(self) -> None:
+        """Takes the staged logits of the last captured step (whose stream
+        has been waited for since) into the result."""
+        if self._staged is not None:
+            self._decode_logits.append(self._staged.clone())
+            self._staged = None
+
+    def _capture(self, st: "_StepBuffers", side: torch.cuda.Stream) -> torch.cuda.CUDAGraph:
+        """The step captured on the stream its eager run warmed up. Cached
+        device memory is given back first only where less than CAPTURE_FREE
+        is left: it takes 3 ms, and the next prefill allocates it anew."""
+        torch.cuda.synchronize(self.device)
+        if torch.cuda.mem_get_info(self.device)[0] < CAPTURE_FREE:
+            torch.cuda.empty_cache()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(side):
+            graph.capture_begin()
+            try:
+                self._graph_body(st)
+            finally:
+                graph.capture_end()
+        return graph
 
     def _graph_body(self, st: "_StepBuffers") -> None:
         bs = self.cache.layout.block_size
@@ -593,6 +633,7 @@ class LlamaPagedDecodeRunner:
             next_tokens = torch.stack([s[0] for s in sampled])
         positions = [r.prompt_tokens + r.generated_tokens for r in requests]
         logits = self._forward_decode(next_tokens, requests, positions)
+        self._collect_logits()
         self._decode_logits.append(used.float().cpu())
         toks = next_tokens.tolist()
         for i, r in enumerate(requests):
@@ -630,6 +671,7 @@ class LlamaPagedDecodeRunner:
                     decode_steps.append(ms)
                 else:
                     raise RuntimeError("scheduler became idle before all requests finished")
+        self._collect_logits()
         if len(self._prompt_logits) != len(self.requests):
             raise RuntimeError("prefill did not produce one final logits tensor per request")
         generated = tuple(tuple(self._generated[r.request_id]) for r in self.requests)

@@ -126,3 +126,26 @@ def test_what_the_kernels_do_not_restate_is_left_to_the_module():
         torch.nn.utils.parametrizations.weight_norm(lin)
         assert not lo.linear_fits(lin, x)
     assert not lo.kernels_apply(x)  # autograd may record
+
+
+def test_a_hooked_head_sees_all_rows_and_gives_the_same_tokens():
+    """The runner computes logits of the chunks' last rows only; with a hook
+    on the head, of all rows. Ragged prompts, two prefill batches."""
+    from inferkernellab_amd.llama import LlamaConfig, LlamaPagedDecodeRunner, random_llama
+
+    cfg = LlamaConfig(vocab_size=128, hidden_size=256, intermediate_size=512, num_hidden_layers=2,
+                      num_attention_heads=4, num_key_value_heads=2)
+    model = random_llama(cfg, seed=3, device="cuda", dtype=torch.float32)
+    prompts = [list(range(1, 1 + n)) for n in (5, 17, 9, 30)]
+    kw = dict(max_new_tokens=4, max_num_batched_tokens=32)
+    plain = LlamaPagedDecodeRunner(model, prompts, **kw).run()
+    rows = []
+    handle = model.lm_head.register_forward_hook(lambda mod, args, out: rows.append(args[0].shape))
+    hooked = LlamaPagedDecodeRunner(model, prompts, **kw).run()
+    handle.remove()
+    assert any(len(shape) == 3 for shape in rows)
+    assert plain.generated_tokens == hooked.generated_tokens
+    assert torch.allclose(plain.prompt_logits, hooked.prompt_logits, atol=1e-5, rtol=1e-5)
+    assert len(plain.decode_logits) == len(hooked.decode_logits) == 4
+    for a, b in zip(plain.decode_logits, hooked.decode_logits):
+        assert a.shape == b.shape and not a.is_cuda and torch.allclose(a, b, atol=1e-5, rtol=1e-5)
