@@ -12,10 +12,16 @@
 // is exact in fp32, so doing the same three roundings here reproduces it;
 // fp32 tensors round each product before the add for the same reason.
 //
-// Layout: one workgroup per token; each thread takes 16-byte chunk c of the
-// first half of a q or k row together with chunk c of the second half
-// (rotate-half pairs element i with element i +- D/2), and v rows are
-// copied in 16-byte chunks. Slots outside the cache are skipped.
+// Layout: one workgroup per token (up to SPREAD_TOKENS tokens, one per 256 of
+// its items); each thread takes 16-byte chunk c of the first half of a q or k
+// row together with chunk c of the second half (rotate-half pairs element i
+// with element i +- D/2), and v rows are copied in 16-byte chunks. The token
+// is uniform in a workgroup, so its slot and row addresses are scalar: items
+// numbered over all tokens took 30.3 us at 4096 tokens (32/8 heads of 128,
+// bf16) against 28.7. Bound: memory; at few tokens the launch and one round
+// trip, which is why a thread takes no second item there (16 tokens 4.8 ->
+// 3.7 us, 32/32 heads 5.6 -> 3.6). Slots outside the cache are skipped.
+#include "fp8_row.h"
 #include "ikl_common.h"
 
 namespace ikl {
@@ -127,7 +133,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeParams p) {
   // rows: num_heads q rows, then num_kv_heads k rows (rotated); then v rows (copied)
   const int rot_items = (p.num_heads + p.num_kv_heads) * hc;
   const int copy_items = p.num_kv_heads * 2 * hc;
-  for (int i = threadIdx.x; i < rot_items + copy_items; i += blockDim.x) {
+  for (int i = threadIdx.x + blockIdx.y * blockDim.x; i < rot_items + copy_items; i += blockDim.x * gridDim.y) {
     if (i < rot_items) {
       const int row = i / hc, c = i - row * hc;
       const u32x4 cl = load16(crow + c * 16), ch = load16(crow + (c + hc) * 16);
@@ -157,12 +163,15 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeParams p) {
 }
 
 // ------------------------------------------------------ into an FP8 cache
-// One wave per row of a token: q rows (rotated), k rows (rotated, then
-// quantised) and v rows (quantised). Lane l takes elements 4l .. 4l+3 of
-// the first half and their rotate-half partners 4l + D/2 ..; the k / v row
-// maximum gives the power-of-two scale e4m3_row_scale(amax) and codes
-// e4m3(x / scale), as ikl_append_kv does for rows that arrive already
-// rotated.
+// LPR lanes per row of a token, as many as its octets need (a power of two):
+// q rows (rotated), k rows (rotated, then quantised) and v rows (quantised).
+// Lane l of a row takes elements 4l .. 4l+3 of the first half and their
+// rotate-half partners 4l + D/2 ..; the k / v row maximum gives the
+// power-of-two scale e4m3_row_scale(amax) and codes e4m3(x / scale), as
+// ikl_append_kv does for rows that arrive already rotated. Bound: memory; a
+// one-wave workgroup per row used 16 of 64 lanes at 128 dims and ran at the
+// dispatcher's rate (4096 tokens, 32/8 heads of 128, bf16: 91 us, packed 30 us
+// or 3.1 TB/s; 512 tokens 14.7 -> 6.8).
 struct RopeFp8Params {
   RopeParams r;  // kc / vc strides in bytes (= elements)
   float *k_scale;
@@ -216,103 +225,101 @@ struct four<f32_tag> {
   }
 };
 
-__device__ inline float wave_max_abs(float v) {
-  v = fmaxf(v, dpp_mov<DPP_QUAD_XOR1>(v));
-  v = fmaxf(v, dpp_mov<DPP_QUAD_XOR2>(v));
-  v = fmaxf(v, dpp_mov<DPP_ROW_HALF_MIRROR>(v));
-  v = fmaxf(v, dpp_mov<DPP_ROW_MIRROR>(v));
-  return max_xor32(max_xor16(v));
-}
-
-// Quantises 8 values (lo[4] at element 4l, hi[4] at 4l + D/2) of a row whose
-// wave-wide maximum magnitude is amax; writes codes and (lane 0) the scale.
-__device__ inline void store_fp8_row(char *dst, float *scale_dst, int lane, int half, bool on, const float *lo,
-                                     const float *hi, float amax) {
-  const float scale = e4m3_row_scale(amax);
-  float y[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    y[i] = fminf(fmaxf(lo[i] / scale, -448.0f), 448.0f);
-    y[4 + i] = fminf(fmaxf(hi[i] / scale, -448.0f), 448.0f);
-  }
-  int wl = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
-  wl = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], wl, true);
-  int wh = __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], 0, false);
-  wh = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], wh, true);
-  if (on) {
-    *reinterpret_cast<int *>(dst + 4 * lane) = wl;
-    *reinterpret_cast<int *>(dst + half + 4 * lane) = wh;
-  }
-  if (lane == 0) *scale_dst = scale;
-}
-
-template <typename Tag, typename IdxT>
-__global__ __launch_bounds__(64) void rope_append_fp8_kernel(RopeFp8Params f) {
+template <typename Tag, typename IdxT, int LPR>
+__global__ __launch_bounds__(256) void rope_append_fp8_kernel(RopeFp8Params f) {
   using M = rope_math<Tag>;
   using F = four<Tag>;
   constexpr int EB = F::BYTES / 4;
   const RopeParams &p = f.r;
-  const int lane = threadIdx.x;
-  const int row = blockIdx.x;  // q rows, then k rows, then v rows
-  const int64_t t = blockIdx.y;
+  const int lane = threadIdx.x % LPR;
+  const int64_t t = blockIdx.x;
+  const int rows = p.num_heads + 2 * p.num_kv_heads;  // q rows, then k rows, then v rows
   const int half = f.head_dim / 2;
   const bool on = 4 * lane < half;
   const int64_t slot = (int64_t)reinterpret_cast<const IdxT *>(p.slots)[t];
   const bool slot_ok = slot >= 0 && slot < p.num_slots;
   const int64_t blk = slot_ok ? slot / p.block_size : 0;
   const int64_t off = slot_ok ? slot - blk * p.block_size : 0;
-  if (row >= p.num_heads && !slot_ok) return;
-  const int kv_row = row - p.num_heads;
-  float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
-  if (kv_row >= p.num_kv_heads) {  // v row: quantise as is
-    const int h = kv_row - p.num_kv_heads;
-    const char *src = p.value + t * p.v_st + h * p.v_sh;
+  // every lane of a wave makes the same passes: the maximum crosses lanes
+  for (int r0 = blockIdx.y * (256 / LPR); r0 < rows; r0 += gridDim.y * (256 / LPR)) {
+    const int want = r0 + threadIdx.x / LPR;
+    const bool has = want < rows;
+    const int row = has ? want : rows - 1;  // groups past the last row read it again
+    const int kv_row = row - p.num_heads;
+    const bool is_q = kv_row < 0, is_v = kv_row >= p.num_kv_heads;
+    const int h = is_q ? row : is_v ? kv_row - p.num_kv_heads : kv_row;
+    float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
     if (on) {
+      const char *src = is_q ? p.q_in + t * p.qi_st + h * p.qi_sh
+                             : is_v ? p.value + t * p.v_st + h * p.v_sh : p.key + t * p.k_st + h * p.k_sh;
       F::load(src + 4 * lane * EB, a);
       F::load(src + (half + 4 * lane) * EB, b);
+      if (!is_v) {
+        float x1[4], x2[4], c1[4], c2[4], s1[4], s2[4];
+        F::load(p.cos + t * p.cos_st + 4 * lane * EB, c1);
+        F::load(p.cos + t * p.cos_st + (half + 4 * lane) * EB, c2);
+        F::load(p.sin + t * p.sin_st + 4 * lane * EB, s1);
+        F::load(p.sin + t * p.sin_st + (half + 4 * lane) * EB, s2);
+  #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x1[i] = a[i];
+          x2[i] = b[i];
+          a[i] = M::add(M::mul(x1[i], c1[i]), M::mul(-x2[i], s1[i]));  // x1 cos - x2 sin
+          b[i] = M::add(M::mul(x2[i], c2[i]), M::mul(x1[i], s2[i]));   // x2 cos + x1 sin
+        }
+      }
     }
-    float m = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m = fmaxf(m, fmaxf(fabsf(a[i]), fabsf(b[i])));
-    store_fp8_row(p.vc + blk * p.vc_sb + off * p.vc_st + h * p.vc_sh, f.v_scale + blk * f.s_sb + h * f.s_sh + off,
-                  lane, half, on, a, b, wave_max_abs(m));
-    return;
-  }
-  // rotate a q or k row
-  const char *src = row < p.num_heads ? p.q_in + t * p.qi_st + row * p.qi_sh : p.key + t * p.k_st + kv_row * p.k_sh;
-  float x1[4] = {0.f, 0.f, 0.f, 0.f}, x2[4] = {0.f, 0.f, 0.f, 0.f}, c1[4], c2[4], s1[4], s2[4];
-  if (on) {
-    F::load(src + 4 * lane * EB, x1);
-    F::load(src + (half + 4 * lane) * EB, x2);
-    F::load(p.cos + t * p.cos_st + 4 * lane * EB, c1);
-    F::load(p.cos + t * p.cos_st + (half + 4 * lane) * EB, c2);
-    F::load(p.sin + t * p.sin_st + 4 * lane * EB, s1);
-    F::load(p.sin + t * p.sin_st + (half + 4 * lane) * EB, s2);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] = M::add(M::mul(x1[i], c1[i]), M::mul(-x2[i], s1[i]));  // x1 cos - x2 sin
-      b[i] = M::add(M::mul(x2[i], c2[i]), M::mul(x1[i], s2[i]));   // x2 cos + x1 sin
-    }
-  }
-  if (row < p.num_heads) {
-    if (on) {
-      char *dst = p.q_out + t * p.qo_st + row * p.qo_sh;
+    if (is_q && has && on) {
+      char *dst = p.q_out + t * p.qo_st + h * p.qo_sh;
       F::store(dst + 4 * lane * EB, a);
       F::store(dst + (half + 4 * lane) * EB, b);
     }
-    return;
+    if (__builtin_amdgcn_ballot_w64(!is_q) == 0ull) continue;  // no k or v row in this wave
+    float m = 0.f;
+  #pragma unroll
+    for (int i = 0; i < 4; ++i) m = fmaxf(m, fmaxf(fabsf(a[i]), fabsf(b[i])));
+    const float scale = e4m3_row_scale(group_max<LPR>(m));
+    if (is_q || !has || !slot_ok) continue;
+    char *dst = is_v ? p.vc + blk * p.vc_sb + off * p.vc_st + h * p.vc_sh
+                     : p.kc + blk * p.kc_sb + off * p.kc_st + h * p.kc_sh;
+    if (on) {
+      *reinterpret_cast<int *>(dst + 4 * lane) = fp8x4(a, scale);
+      *reinterpret_cast<int *>(dst + half + 4 * lane) = fp8x4(b, scale);
+    }
+    if (lane == 0) (is_v ? f.v_scale : f.k_scale)[blk * f.s_sb + h * f.s_sh + off] = scale;
   }
-  float m = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m = fmaxf(m, fmaxf(fabsf(a[i]), fabsf(b[i])));
-  store_fp8_row(p.kc + blk * p.kc_sb + off * p.kc_st + kv_row * p.kc_sh,
-                f.k_scale + blk * f.s_sb + kv_row * f.s_sh + off, lane, half, on, a, b, wave_max_abs(m));
+}
+
+// Up to this many tokens a token's items spread over workgroups of one pass.
+constexpr int64_t SPREAD_TOKENS = 1024;
+
+// `items` of a token in workgroups of `per`
+dim3 token_grid(int64_t tokens, int64_t items, int64_t per) {
+  const int64_t parts = tokens <= SPREAD_TOKENS ? (items + per - 1) / per : 1;
+  return dim3((unsigned)tokens, (unsigned)(parts < 65535 ? parts : 65535));
 }
 
 template <typename Tag>
 void launch_rope(const RopeParams &p, int64_t tokens, bool i64, hipStream_t s) {
-  if (i64) rope_append_kernel<Tag, int64_t><<<dim3((unsigned)tokens), 256, 0, s>>>(p);
-  else rope_append_kernel<Tag, int32_t><<<dim3((unsigned)tokens), 256, 0, s>>>(p);
+  const dim3 grid = token_grid(tokens, (p.num_heads + 3 * (int64_t)p.num_kv_heads) * p.half_chunks, 256);
+  if (i64) rope_append_kernel<Tag, int64_t><<<grid, 256, 0, s>>>(p);
+  else rope_append_kernel<Tag, int32_t><<<grid, 256, 0, s>>>(p);
+}
+
+template <typename Tag, int LPR>
+void launch_rope_fp8(const RopeFp8Params &f, int64_t tokens, bool i64, hipStream_t s) {
+  const dim3 grid = token_grid(tokens, f.r.num_heads + 2 * (int64_t)f.r.num_kv_heads, 256 / LPR);
+  if (i64) rope_append_fp8_kernel<Tag, int64_t, LPR><<<grid, 256, 0, s>>>(f);
+  else rope_append_fp8_kernel<Tag, int32_t, LPR><<<grid, 256, 0, s>>>(f);
+}
+
+template <typename Tag>
+void launch_rope_fp8(const RopeFp8Params &f, int64_t tokens, bool i64, hipStream_t s) {
+  const int octets = f.head_dim / 8;
+  if (octets <= 8) launch_rope_fp8<Tag, 8>(f, tokens, i64, s);
+  else if (octets <= 16) launch_rope_fp8<Tag, 16>(f, tokens, i64, s);
+  else if (octets <= 32) launch_rope_fp8<Tag, 32>(f, tokens, i64, s);
+  else launch_rope_fp8<Tag, 64>(f, tokens, i64, s);
 }
 
 bool al16(const void *ptr) { return ((uintptr_t)ptr & 15u) == 0; }
@@ -404,18 +411,11 @@ extern "C" int ikl_rope_append_kv(const ikl_rope_append_args *a, void *stream) {
     f.s_sb = a->scale_stride_block;
     f.s_sh = a->scale_stride_head;
     f.head_dim = a->head_dim;
-    const dim3 grid((unsigned)(a->num_heads + 2 * a->num_kv_heads), (unsigned)a->num_tokens);
-#define IKL_ROPE8(TAG)                                                                  \
-  do {                                                                                  \
-    if (i64) rope_append_fp8_kernel<TAG, int64_t><<<grid, 64, 0, s>>>(f);               \
-    else rope_append_fp8_kernel<TAG, int32_t><<<grid, 64, 0, s>>>(f);                   \
-  } while (0)
     switch (a->dtype) {
-      case IKL_F16: IKL_ROPE8(f16_tag); break;
-      case IKL_BF16: IKL_ROPE8(bf16_tag); break;
-      default: IKL_ROPE8(f32_tag); break;
+      case IKL_F16: launch_rope_fp8<f16_tag>(f, a->num_tokens, i64, s); break;
+      case IKL_BF16: launch_rope_fp8<bf16_tag>(f, a->num_tokens, i64, s); break;
+      default: launch_rope_fp8<f32_tag>(f, a->num_tokens, i64, s); break;
     }
-#undef IKL_ROPE8
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(IKL_ELAUNCH, std::string("rope append launch: ") + hipGetErrorString(e));
     return IKL_OK;
