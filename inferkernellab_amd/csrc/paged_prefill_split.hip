@@ -13,14 +13,15 @@
 // 0.7 us at KG = 1, times the steps of the longest workgroup. So the loop
 // favours few instructions (32x32x16 MFMAs: half as many, one softmax row per
 // lane, 8 dot products for the denominators) and runs the next tile's QK^T
-// under this one's exponentials. 12 % fewer cycles than the 16x16x32 loop on
-// such launches; where a launch fills the chip and meets its power limit the
-// clock falls by more than that, which is why the other kernel stays.
+// under this one's exponentials. 9 % fewer cycles than the 16x16x32 loop on
+// the ragged chunks below. At 8 x 4096 it is 6.5 % fewer (2.69 -> 2.52 M), but
+// that launch meets the power limit: the clock falls from 2155 to 2042 MHz
+// and it takes 1173-1206 us against 1160, which is why the other kernel stays.
 //
 // 32/8 heads of 128, bf16, against paged_prefill_mfma_kernel: 4 requests x
 // (2000 + 64 tokens) 57.6 -> 28.9 us, 1 x 1024 tokens 32.1 -> 23.8, 2 x 1024
 // 36.6 -> 32.8; 4 ragged chunks (1024-3072 + 517-1024) over the FP8 cache
-// 220 -> 202.
+// 222 -> 205.
 #include "ikl_common.h"
 #include "mfma_ops.h"
 #include "paged_attn.h"
