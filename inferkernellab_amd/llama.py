@@ -312,20 +312,22 @@ class LlamaPagedDecodeRunner:
         else:
             ops.append_kv_hip(key.contiguous(), value.contiguous(), self.cache, slots, layer=layer)
 
-    def _add_norm(self, norm, hidden: torch.Tensor, delta: torch.Tensor | None, *, packed: bool = False):
-        """(hidden + delta, norm of it): one kernel for a plain RMSNorm.
-        `packed`: (norm, rows) for decode_linear, the norm in operand order
-        (rows set) where the kernel runs."""
-        if (layer_ops.plain_module(norm, RMSNorm) and layer_ops.kernels_apply(hidden)
+    def _norm_restated(self, norm, hidden: torch.Tensor, delta: torch.Tensor | None) -> bool:
+        """Whether the kernel runs hidden + delta and the norm of it."""
+        return (layer_ops.plain_module(norm, RMSNorm) and layer_ops.kernels_apply(hidden)
                 and (delta is None or (type(delta) is torch.Tensor and delta.dtype == hidden.dtype
                                        and delta.shape == hidden.shape and delta.device == hidden.device))
-                and layer_ops.norm_fits(norm.weight, hidden)):
-            hidden, x = layer_ops.add_rms_norm(hidden, delta, norm.weight, norm.variance_epsilon, packed=packed)
-            return hidden, (x, hidden.shape[0]) if packed else x
+                and layer_ops.norm_fits(norm.weight, hidden))
+
+    def _add_norm(self, norm, hidden: torch.Tensor, delta: torch.Tensor | None, *, packed: bool = False):
+        """(hidden + delta, norm of it): one kernel for a plain RMSNorm.
+        `packed` (of a layer that _decode_linears accepts): the norm in
+        operand order, for decode_linear."""
+        if packed or self._norm_restated(norm, hidden, delta):
+            return layer_ops.add_rms_norm(hidden, delta, norm.weight, norm.variance_epsilon, packed=packed)
         if delta is not None:
             hidden = hidden + delta
-        x = norm(hidden)
-        return hidden, (x, None) if packed else x
+        return hidden, norm(hidden)
 
     def _mlp(self, mlp, x: torch.Tensor) -> torch.Tensor:
         gate, up = mlp.gate_proj(x), mlp.up_proj(x)
@@ -334,12 +336,15 @@ class LlamaPagedDecodeRunner:
             return mlp.down_proj(layer_ops.silu_mul(gate, up))
         return mlp.down_proj(mlp.act_fn(gate) * up)
 
-    def _decode_linears(self, layer, hidden: torch.Tensor) -> bool:
+    def _decode_linears(self, layer, hidden: torch.Tensor, delta: torch.Tensor | None) -> bool:
         """Whether the decode linear kernels restate this layer's linears and
-        activation on `hidden`: the q/k/v projections, the o projection and
-        its residual add, the gated MLP and its."""
+        activation on `hidden` + `delta`: the q/k/v projections, the o
+        projection and its residual add, the gated MLP and its. They read the
+        norms in the norm kernel's layout, so both norms have to be restated:
+        a module's result may have any type and strides."""
         att, mlp = layer.self_attn, layer.mlp
-        return (layer_ops.kernels_apply(hidden)
+        return (self._norm_restated(layer.input_layernorm, hidden, delta)
+                and self._norm_restated(layer.post_attention_layernorm, hidden, None)
                 and all(layer_ops.linear_fits(p, hidden)
                         for p in (att.q_proj, att.k_proj, att.v_proj, mlp.gate_proj, mlp.up_proj))
                 and layer_ops.plain_module(mlp.act_fn, nn.SiLU) and not mlp.act_fn.inplace
@@ -372,12 +377,11 @@ class LlamaPagedDecodeRunner:
         delta = None  # the last block's output, not yet added to `hidden`
         for li, layer in enumerate(m.layers):
             att = layer.self_attn
-            kernels = self._decode_linears(layer, hidden)
+            kernels = self._decode_linears(layer, hidden, delta)
             hidden, x = self._add_norm(layer.input_layernorm, hidden, delta, packed=kernels)
             delta = None
             if kernels:
-                q, k, v = layer_ops.decode_linear(x[0], (att.q_proj.weight, att.k_proj.weight, att.v_proj.weight),
-                                                  rows=x[1])
+                q, k, v = layer_ops.decode_linear(x, (att.q_proj.weight, att.k_proj.weight, att.v_proj.weight), rows=n)
             else:
                 q, k, v = att.q_proj(x), att.k_proj(x), att.v_proj(x)
             q = q.view(n, self.num_heads, self.head_dim)
@@ -394,7 +398,7 @@ class LlamaPagedDecodeRunner:
             if kernels:
                 hidden = layer_ops.decode_linear(o, (att.o_proj.weight,), residual=hidden)
                 _, x = self._add_norm(layer.post_attention_layernorm, hidden, None, packed=True)
-                x = layer_ops.decode_linear(x[0], (layer.mlp.gate_proj.weight, layer.mlp.up_proj.weight), rows=x[1],
+                x = layer_ops.decode_linear(x, (layer.mlp.gate_proj.weight, layer.mlp.up_proj.weight), rows=n,
                                             silu=True, packed=True)
                 hidden = layer_ops.decode_linear(x, (layer.mlp.down_proj.weight,), rows=n, residual=hidden)
             else:
