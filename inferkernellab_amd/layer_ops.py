@@ -100,8 +100,8 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tens
     total = x
     if delta is not None:
         d = _flat_rows(delta)
-        if d is None:
-            d = delta.contiguous().view(-1, delta.shape[-1])
+        if d is None:  # also a contiguous one at an odd address
+            d = delta.clone(memory_format=torch.contiguous_format).view(-1, delta.shape[-1])
         total = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         a.delta, a.delta_stride = d.data_ptr(), d.stride(0)
         a.sum, a.sum_stride = total.data_ptr(), x.shape[-1]

@@ -45,6 +45,20 @@ def test_add_rms_norm(dtype, rows, cols, add):
     _close(out, _norm(expected, w, 1e-6), dtype, 2, 1e-3)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_add_rms_norm_takes_a_delta_at_any_address(dtype):
+    from inferkernellab_amd import layer_ops as lo
+
+    x = torch.randn(5, 64, device="cuda").to(dtype)
+    delta = torch.randn(5 * 64 + 1, device="cuda").to(dtype)[1:].view(5, 64)
+    w = torch.ones(64, device="cuda", dtype=dtype)
+    assert delta.is_contiguous() and delta.data_ptr() % 16
+    with torch.no_grad():
+        total, out = lo.add_rms_norm(x, delta, w, 1e-6)
+    assert torch.equal(total, x + delta)
+    _close(out, _norm(x + delta, w, 1e-6), dtype, 2, 1e-3)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [(8,), (3, 40), (257, 512)])
 def test_silu_mul(dtype, shape):
