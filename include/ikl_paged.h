@@ -322,7 +322,8 @@ int32_t ikl_check_metadata(const void *tables, int32_t table_type, int64_t table
 
 /* Waits for the `count` words of a check enqueued on `stream` (work enqueued
  * after it is not waited for) and returns its findings, or a negative IKL_E*
- * code when the launch failed. */
+ * code when the launch failed. The device of the stream has to be current, as
+ * for the check: the default stream's handle alone does not name it. */
 int32_t ikl_check_metadata_wait(const uint32_t *flags, int32_t count, void *stream);
 
 /* RMSNorm of x [rows, cols] (row strides in elements, rows 16-byte aligned),

@@ -146,9 +146,9 @@ class _MetadataCheck:
         flags = getattr(_check_flags, "words", None)
         if flags is None:
             flags = _check_flags.words = torch.empty(_CHECK_WORDS, dtype=torch.int32, pin_memory=True)
-        device = context_lens.device
-        with _on_device(device):
-            self._stream = torch.cuda.current_stream(device).cuda_stream
+        self._device = context_lens.device
+        with _on_device(self._device):
+            self._stream = torch.cuda.current_stream(self._device).cuda_stream
             self._flags = flags.data_ptr()
             self._count = self._lib.ikl_check_metadata(
                 block_tables.data_ptr(), _INDEX_TYPES[block_tables.dtype], block_tables.stride(0),
@@ -161,7 +161,9 @@ class _MetadataCheck:
         count, self._count = self._count, 0
         if count <= 0:
             return
-        found = self._lib.ikl_check_metadata_wait(self._flags, count, self._stream)
+        # the default stream's handle names the current device's stream
+        with _on_device(self._device):
+            found = self._lib.ikl_check_metadata_wait(self._flags, count, self._stream)
         if found < 0:
             _check_flags.words = None
             _lib.check(found, "check metadata")
