@@ -26,7 +26,6 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
-import threading
 
 import torch
 
@@ -125,14 +124,34 @@ def _on_device(device: torch.device):
     return torch.cuda.device(device)
 
 
-_check_flags = threading.local()  # one pinned buffer a thread: a check is waited for before the next begins
+# Pinned words for the value checks. A buffer serves one check at a time and is
+# free again once that check has been waited for; one whose wait never came (an
+# asynchronous exception between the two) or failed stays taken: its kernel may
+# write it late. All are kept here, so none returns to the host allocator.
 _CHECK_WORDS = 64
+_check_words_made: list = []
+_check_words_free: list = []
 _CHECK_MESSAGES = (  # in the order of triton_ops.py:439-457
     (_lib.IKL_CHECK_LENGTH_POSITIVE, "context lengths must be positive"),
     (_lib.IKL_CHECK_LENGTH_CAPACITY, "context length exceeds block table capacity"),
     (_lib.IKL_CHECK_BLOCK_ID, "block table contains an invalid physical block id"),
     (_lib.IKL_CHECK_LENGTH_MAX, "context length exceeds max_context_len"),
 )
+
+
+def _pinned_words() -> torch.Tensor:
+    return torch.empty(_CHECK_WORDS, dtype=torch.int32, pin_memory=True)
+
+
+def _take_check_words():
+    """Words no check is in flight on, as a ctypes array over pinned memory."""
+    try:
+        return _check_words_free.pop()
+    except IndexError:
+        tensor = _pinned_words()
+        words = (ctypes.c_uint32 * _CHECK_WORDS).from_address(tensor.data_ptr())
+        _check_words_made.append((tensor, words))
+        return words
 
 
 class _MetadataCheck:
@@ -143,18 +162,20 @@ class _MetadataCheck:
 
     def __init__(self, block_tables, context_lens, layout, max_context_len):
         self._lib = _require_backend()
-        flags = getattr(_check_flags, "words", None)
-        if flags is None:
-            flags = _check_flags.words = torch.empty(_CHECK_WORDS, dtype=torch.int32, pin_memory=True)
         self._device = context_lens.device
+        self._words = _take_check_words()
+        self._words[0] = 0  # marked as pending just before the kernel is launched
+        self._count = 0
         with _on_device(self._device):
             self._stream = torch.cuda.current_stream(self._device).cuda_stream
-            self._flags = flags.data_ptr()
             self._count = self._lib.ikl_check_metadata(
                 block_tables.data_ptr(), _INDEX_TYPES[block_tables.dtype], block_tables.stride(0),
                 block_tables.stride(1), context_lens.data_ptr(), _INDEX_TYPES[context_lens.dtype],
                 context_lens.stride(0), block_tables.shape[0], block_tables.shape[1], layout.block_size,
-                layout.num_blocks, int(max_context_len or 0), self._flags, _CHECK_WORDS, self._stream)
+                layout.num_blocks, int(max_context_len or 0), ctypes.addressof(self._words), _CHECK_WORDS,
+                self._stream)
+        if self._count < 0 and self._words[0] == 0:  # refused, nothing was launched
+            _check_words_free.append(self._words)
         _lib.check(min(self._count, 0), "check metadata")
 
     def wait(self) -> None:
@@ -163,10 +184,10 @@ class _MetadataCheck:
             return
         # the default stream's handle names the current device's stream
         with _on_device(self._device):
-            found = self._lib.ikl_check_metadata_wait(self._flags, count, self._stream)
-        if found < 0:
-            _check_flags.words = None
-            _lib.check(found, "check metadata")
+            found = self._lib.ikl_check_metadata_wait(ctypes.addressof(self._words), count, self._stream)
+        if found >= 0:
+            _check_words_free.append(self._words)
+        _lib.check(min(found, 0), "check metadata")
         for bit, message in _CHECK_MESSAGES:
             if found & bit:
                 raise ValueError(message)

@@ -70,3 +70,46 @@ def test_a_check_is_waited_for_on_its_own_device(lib, found):
         with _check():
             assert lib.current == "cuda:0"
     assert [c[:2] for c in lib.calls] == [("check", "cuda:1"), ("wait", "cuda:1")]
+
+
+@pytest.fixture
+def words(monkeypatch):
+    """The module's word buffers, empty, as the test leaves them."""
+    for name in ("_check_words_made", "_check_words_free"):
+        monkeypatch.setattr(ops, name, [], raising=False)
+
+
+def test_words_serve_the_next_check_once_they_were_waited_for(lib, words):
+    for _ in range(3):
+        _check().wait()
+    assert len({c[2] for c in lib.calls}) == 1
+
+
+def test_words_of_a_check_that_was_not_waited_for_are_left_alone(lib, words):
+    """Its kernel may still write: an interrupt came between the two."""
+    lost = _check()
+    _check().wait()
+    with _check():  # and a check that begins while another is in flight
+        _check().wait()
+    first = lib.calls[0][2]
+    assert all(c[2] != first for c in lib.calls[1:])
+    assert lost is not None and any(tensor.data_ptr() == first for tensor, _ in ops._check_words_made)
+
+
+def test_words_of_a_failed_wait_are_kept_and_not_used_again(lib, words):
+    lib.found = -3
+    with pytest.raises(RuntimeError):
+        _check().wait()
+    failed = lib.calls[0][2]
+    lib.found = 0
+    _check().wait()
+    assert lib.calls[-1][2] != failed
+    assert any(tensor.data_ptr() == failed for tensor, _ in ops._check_words_made)
+
+
+def test_words_of_a_refused_check_are_free_again(lib, words, monkeypatch):
+    monkeypatch.setattr(lib, "ikl_check_metadata", lambda *a: -3)
+    for _ in range(3):
+        with pytest.raises(RuntimeError):
+            _check()
+    assert len(ops._check_words_made) == 1
