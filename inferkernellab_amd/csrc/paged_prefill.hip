@@ -577,7 +577,8 @@ hipError_t launch_mfma_dim(int d, const PrefillParams &p, dim3 grid, hipStream_t
       if constexpr (!KV8) paged_prefill_mfma_kernel<Tag, 96, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p);
       else return hipErrorInvalidValue;
       break;
-    default: paged_prefill_mfma_kernel<Tag, 128, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
+    case 128: paged_prefill_mfma_kernel<Tag, 128, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
+    default: return hipErrorInvalidValue;  // no row is wide enough for another width's kernel
   }
   return hipGetLastError();
 }

@@ -490,7 +490,8 @@ hipError_t launch_dim(const PrefillParams &p, hipStream_t s) {
     case 32: paged_prefill_split_kernel<Tag, 32, KG, KV8><<<grid, wg, 0, s>>>(p); break;
     case 64: paged_prefill_split_kernel<Tag, 64, KG, KV8><<<grid, wg, 0, s>>>(p); break;
     case 96: paged_prefill_split_kernel<Tag, 96, KG, KV8><<<grid, wg, 0, s>>>(p); break;
-    default: paged_prefill_split_kernel<Tag, 128, KG, KV8><<<grid, wg, 0, s>>>(p); break;
+    case 128: paged_prefill_split_kernel<Tag, 128, KG, KV8><<<grid, wg, 0, s>>>(p); break;
+    default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
@@ -499,7 +500,8 @@ template <typename Tag>
 hipError_t launch_tag(const PrefillParams &p, int groups, hipStream_t s) {
   if (groups == 1) return p.kv_fp8 ? launch_dim<Tag, 1, true>(p, s) : launch_dim<Tag, 1, false>(p, s);
   if (groups == 2) return p.kv_fp8 ? launch_dim<Tag, 2, true>(p, s) : launch_dim<Tag, 2, false>(p, s);
-  return p.kv_fp8 ? launch_dim<Tag, 4, true>(p, s) : launch_dim<Tag, 4, false>(p, s);
+  if (groups == 4) return p.kv_fp8 ? launch_dim<Tag, 4, true>(p, s) : launch_dim<Tag, 4, false>(p, s);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
