@@ -45,7 +45,9 @@ EXPORTED_SYMBOLS = (
     "ikl_paged_attention_launch_config",
     "ikl_rope_append_kv",
     "ikl_paged_prefill_attention",
+    "ikl_paged_prefill_attention_planned",
     "ikl_paged_prefill_path",
+    "ikl_paged_prefill_plan",
     "ikl_paged_prefill_key_groups",
     "ikl_paged_decode_step",
     "ikl_paged_decode_step_fused",
@@ -329,6 +331,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ikl_rope_append_kv.argtypes = [ctypes.POINTER(RopeAppendArgs), _c_ptr]
     lib.ikl_paged_prefill_attention.restype = ctypes.c_int
     lib.ikl_paged_prefill_attention.argtypes = [ctypes.POINTER(PagedPrefillArgs), _c_ptr]
+    lib.ikl_paged_prefill_attention_planned.restype = ctypes.c_int
+    lib.ikl_paged_prefill_attention_planned.argtypes = [ctypes.POINTER(PagedPrefillArgs), _c_i32, _c_ptr]
+    lib.ikl_paged_prefill_plan.restype = _c_i32
+    lib.ikl_paged_prefill_plan.argtypes = [ctypes.POINTER(PagedPrefillArgs), _c_i64, _c_i64]
     lib.ikl_paged_prefill_key_groups.restype = _c_i32
     lib.ikl_paged_prefill_key_groups.argtypes = [ctypes.POINTER(PagedPrefillArgs)]
     lib.ikl_paged_prefill_path.restype = _c_i32

@@ -570,13 +570,10 @@ __global__ __launch_bounds__(64) void paged_prefill_scalar_kernel(const PrefillP
 
 template <typename Tag, int NG, bool KV8>
 hipError_t launch_mfma_dim(int d, const PrefillParams &p, dim3 grid, hipStream_t s) {
-  // 32 dims, and 96 over the FP8 cache, run the split kernel at every size
   switch (d) {
+    case 32: paged_prefill_mfma_kernel<Tag, 32, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
     case 64: paged_prefill_mfma_kernel<Tag, 64, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
-    case 96:
-      if constexpr (!KV8) paged_prefill_mfma_kernel<Tag, 96, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p);
-      else return hipErrorInvalidValue;
-      break;
+    case 96: paged_prefill_mfma_kernel<Tag, 96, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
     case 128: paged_prefill_mfma_kernel<Tag, 128, NG, KV8><<<grid, 64 * PWAVES, 0, s>>>(p); break;
     default: return hipErrorInvalidValue;  // no row is wide enough for another width's kernel
   }
@@ -591,30 +588,70 @@ bool prefill_mfma_supported(int dtype, int head_dim, int block_size) {
 
 // Waves per row of the split kernel (paged_prefill_split.hip) a launch of the
 // 16-bit matrix cores runs with, or 0 for paged_prefill_mfma_kernel. `blocks`:
-// 128-row workgroups (two are resident per CU, 512 on the chip's 256 CUs).
-// Measured on 32/8 heads, us for 0 / 1 / 2 / 4 (bf16, 128 dims unless said):
-//   a quarter of the CUs: 4 x (2000 + 64 tokens)  57.6 / 51.9 / 36.5 / 28.9
-//   the CUs once:  1 x 1024                       32.1 / 29.3 / 23.8 / 49.7
-//                  8 x (2000 + 128), FP8 cache    64.2 / 58.0 / 54.9 / 123
-//   one resident round: 2 x 1024                  36.6 / 32.8 / 38.3 / -
-// Two rounds gain where the rows sit behind long prefixes (equal, long
-// chains; a table of at least twice the query width stands for that):
-//   4 x (2048 + 517-1024 tokens) 150.7 / 144.8, FP8 cache 166.3 / 152.9,
-//   64 dims 104.0 / 93.9; but 6 x 512 from position 0: 30.5 / 34.4.
-// Beyond that a launch runs at the chip's power limit, where the 16x16x32
-// MFMA is 2-5 % ahead, except for 32 dims (4 x 2048: 78.4 / 66.2) and 96 dims
-// over the FP8 cache (8 x 4096: 1170 / 1091).
-int prefill_key_groups(int64_t blocks, int64_t cap_tokens, int64_t width, int head_dim, bool kv8) {
-  if (blocks <= 64) return 4;
-  if (blocks <= 256) return 2;
-  if (blocks <= 512 || (blocks <= 1024 && cap_tokens >= 2 * width)) return 1;
-  return head_dim == 32 || (head_dim == 96 && kv8) ? 1 : 0;
+// 128-row workgroups, `row_blocks` of them per (request, kv head); two are
+// resident per CU, 512 on the chip's 256 CUs. `longest`: the longest context.
+// Splitting shortens the chain of the longest row, for more copies per
+// product, a longer start and a merge: it pays where the chip is idle and the
+// chain is long. us for 0 / 1 / 2 / 4 waves (bf16, 128 dims, 32/8 heads unless
+// said; requests x tokens from position 0, or behind a prefix):
+//   a quarter of the CUs: 4 x (2000 + 64)     57.6 / 51.9 / 36.5 / 28.9
+//     8 x (480 + 32)                          20.3 / 20.0 / 16.0 / 15.5
+//     but 4 x 32-64                            9.4 / 10.5 / 10.2 / 11.6
+//     2 x (120 + 8)                            8.5 / 8.1 / 8.2 / 9.3
+//   half of them: 4 x 512, 8/2 heads          19.5 / 18.3 / 14.5 / 21.3
+//     8 x 128-256, 8/2 heads                  14.1 / 14.0 / 12.3 / 18.9
+//   the CUs once: 1 x 1024                    32.1 / 29.3 / 23.8 / 49.7
+//     but 8 x 64-128                          12.1 / 13.3 / 14.5 / 35.5
+//     32 x (480 + 32)                         23.1 / 22.1 / 24.9 / 64.7
+//   one resident round: 2 x 1024              36.6 / 32.8 / 38.3 / -
+//     but 8 x 128-256, 32/32 heads            19.9 / 20.7 / 25.8 / -
+//     64 x (480 + 32)                         39.4 / 43.0 / 59.4 / -
+// Up to 96 dims a step costs less against the rest of the launch and the
+// lines lie lower. Chunks behind prefixes of at least their width (`even`)
+// have rows of nearly one length, and the whole chip walks keys to the end:
+// there twice the copies cost more.
+//
+// Two rounds of `even` chunks end part empty. Over 16-bit rows of 128 dims
+// that is worth one wave per row up to a round and a half; with a fuller
+// second round the chip is busy throughout, or the chains are short:
+//   3 x (2048 + 1024) 166 / 150    5 x (512 + 512) 58.5 / 53.6
+//   but 4 x (2048 + 1024) 182 / 187    25 x (128 + 128) 32.1 / 35.9
+// 64 dims gain nothing up to there (3 x (1024 + 1024) 55.3 / 57.2) and past
+// it (4 x (2048 + 1024) 120 / 116), 96 dims and the FP8 cache throughout
+// (4 x (2048 + 512-1024) 151 / 141 and, FP8 at 128 dims, 186 / 173). Beyond
+// two rounds the 16x16x32 MFMA of the other kernel is 2-5 % ahead, except for
+// 32 dims (4 x 2048: 78.4 / 66.2) and 96 dims over the FP8 cache (8 x 4096:
+// 1170 / 1091) with long chains.
+// Over 3700 shapes around these lines no plan is more than 5 % behind kernel 0
+// and 8 are more than 3 % behind; on the average they are 5.9 % ahead.
+int prefill_key_groups(int64_t blocks, int64_t row_blocks, int64_t longest, bool even, int head_dim, bool kv8) {
+  const bool narrow = head_dim <= 96;
+  if (blocks <= 64 && longest >= (narrow ? 128 : 256)) return 4;
+  if (blocks <= 128 && longest >= (narrow ? 160 : 192)) return 2;
+  if (blocks <= 256 && longest >= (even ? 1024 : 320)) return 2;
+  if (blocks <= 512) return longest >= (even ? 1024 : head_dim <= 64 ? 257 : 512) ? 1 : 0;
+  if (longest < 1024 || row_blocks < 2) return 0;
+  if (head_dim == 32 || (head_dim == 96 && kv8)) return 1;
+  if (blocks > 1024 || row_blocks < 3 || !even) return 0;
+  return head_dim == 64 ? blocks > 768 : head_dim == 96 || kv8 || blocks <= 768;
 }
 
-int64_t prefill_blocks(const ikl_paged_prefill_args *a) {
+int64_t prefill_row_blocks(const ikl_paged_prefill_args *a) {
   const int64_t rows = a->query_width * (a->num_heads / a->num_kv_heads);
   constexpr int64_t rows_per_wg = 16 * PREFILL_NG * PWAVES;  // RWG of the kernel
-  return (rows + rows_per_wg - 1) / rows_per_wg * ((a->batch * a->num_kv_heads + 7) / 8 * 8);
+  return (rows + rows_per_wg - 1) / rows_per_wg;
+}
+
+int64_t prefill_bh_pad(const ikl_paged_prefill_args *a) { return (a->batch * a->num_kv_heads + 7) / 8 * 8; }
+
+// The plan of a launch of the matrix-core family. A caller that does not know
+// its ranges (0) most likely has a request that fills the query width, so its
+// longest context is taken to be that, from position 0.
+int prefill_plan(const ikl_paged_prefill_args *a, int64_t longest_context, int64_t shortest_start) {
+  const int64_t row_blocks = prefill_row_blocks(a);
+  return prefill_key_groups(row_blocks * prefill_bh_pad(a), row_blocks,
+                            longest_context > 0 ? longest_context : a->query_width,
+                            shortest_start >= a->query_width, a->head_dim, a->cache_dtype == IKL_FP8_E4M3);
 }
 
 bool aligned(const void *ptr, int64_t bytes) { return ((uintptr_t)ptr) % bytes == 0; }
@@ -628,15 +665,24 @@ extern "C" int32_t ikl_paged_prefill_path(int32_t dtype, int32_t head_dim, int32
   return prefill_mfma_supported(dtype, head_dim, block_size) ? IKL_PATH_MFMA_GROUPED : IKL_PATH_SCALAR_GROUPED;
 }
 
-extern "C" int32_t ikl_paged_prefill_key_groups(const ikl_paged_prefill_args *a) {
-  if (!a || a->batch <= 0 || a->query_width <= 0 || a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0)
-    return fail(IKL_EINVAL, "ikl_paged_prefill_key_groups: invalid arguments");
+extern "C" int32_t ikl_paged_prefill_plan(const ikl_paged_prefill_args *a, int64_t longest_context,
+                                          int64_t shortest_start) {
+  if (!a || a->batch <= 0 || a->query_width <= 0 || a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0 ||
+      longest_context < 0 || shortest_start < 0)
+    return fail(IKL_EINVAL, "ikl_paged_prefill_plan: invalid arguments");
   if (!prefill_mfma_supported(a->dtype, a->head_dim, a->block_size) || a->path == IKL_PATH_SCALAR_GROUPED) return 0;
-  return prefill_key_groups(prefill_blocks(a), a->table_width * a->block_size, a->query_width, a->head_dim,
-                            a->cache_dtype == IKL_FP8_E4M3);
+  return prefill_plan(a, longest_context, shortest_start);
 }
 
-extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void *stream) {
+extern "C" int32_t ikl_paged_prefill_key_groups(const ikl_paged_prefill_args *a) {
+  return ikl_paged_prefill_plan(a, 0, 0);
+}
+
+extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *args, void *stream) {
+  return ikl_paged_prefill_attention_planned(args, IKL_PREFILL_AUTO, stream);
+}
+
+extern "C" int ikl_paged_prefill_attention_planned(const ikl_paged_prefill_args *a, int32_t plan, void *stream) {
   if (!a) return fail(IKL_EINVAL, "ikl_paged_prefill_attention: args is NULL");
   if (a->batch <= 0 || a->query_width <= 0 || a->num_heads <= 0 || a->num_kv_heads <= 0 || a->head_dim <= 0 ||
       a->block_size <= 0 || a->num_blocks <= 0 || a->table_width <= 0)
@@ -668,6 +714,9 @@ extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void
   const int ceb = kv8 ? 1 : eb;  // cache bytes per element
   if (path != IKL_PATH_MFMA_GROUPED && path != IKL_PATH_SCALAR_GROUPED)
     return fail(IKL_EINVAL, "ikl_paged_prefill_attention: path must be -1, IKL_PATH_SCALAR_GROUPED or IKL_PATH_MFMA_GROUPED");
+  if (plan != IKL_PREFILL_AUTO && plan != 0 &&
+      (path != IKL_PATH_MFMA_GROUPED || (plan != 1 && plan != 2 && plan != 4)))
+    return fail(IKL_EINVAL, "ikl_paged_prefill_attention: plan must be -1, 0 or, on the matrix-core path, 1, 2 or 4");
   if (path == IKL_PATH_MFMA_GROUPED && auto_path != IKL_PATH_MFMA_GROUPED)
     return fail(IKL_EUNSUPPORTED, "ikl_paged_prefill_attention: no MFMA kernel for this dtype / head_dim / block_size");
   if (path == IKL_PATH_MFMA_GROUPED) {
@@ -744,9 +793,9 @@ extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void
   hipError_t err;
   if (path == IKL_PATH_MFMA_GROUPED) {
     constexpr int NG = PREFILL_NG;
-    const int64_t blocks = prefill_blocks(a);
-    p.bh_pad = (a->batch * a->num_kv_heads + 7) / 8 * 8;
-    p.row_blocks = blocks / p.bh_pad;
+    p.bh_pad = prefill_bh_pad(a);
+    p.row_blocks = prefill_row_blocks(a);
+    const int64_t blocks = p.row_blocks * p.bh_pad;
     // stream-major once a prefix has enough row blocks to fill an XCD's
     // resident workgroups (32 CUs x 2). GQA 32/8 hd128 bf16, 8 x 4096
     // prompts: FETCH_SIZE 3.50 -> 0.67 x the algorithmic bytes, kernel
@@ -755,9 +804,9 @@ extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *a, void
     p.stream_major = p.row_blocks >= 64 && !p.kv_fp8;
     if (blocks > 0x7fffffffLL) return fail(IKL_EINVAL, "ikl_paged_prefill_attention: launch too large");
     const dim3 grid((unsigned)blocks);
-    const int groups = prefill_key_groups(blocks, p.cap_tokens, p.width, p.head_dim, kv8);
-    if (groups > 0)
-      err = launch_prefill_split(p, a->dtype, groups, s);
+    if (plan == IKL_PREFILL_AUTO) plan = prefill_plan(a, 0, 0);
+    if (plan > 0)
+      err = launch_prefill_split(p, a->dtype, plan, s);
     else if (a->dtype == IKL_BF16)
       err = p.kv_fp8 ? launch_mfma_dim<bf16_tag, NG, true>(a->head_dim, p, grid, s)
                      : launch_mfma_dim<bf16_tag, NG, false>(a->head_dim, p, grid, s);

@@ -959,7 +959,7 @@ class PreparedPagedPrefill:
         a.scale = float(scale if scale is not None else layout.head_dim**-0.5)
         a.path = _PATH_IDS[self.path]
         self._args = a
-        self.key_groups = self._lib.ikl_paged_prefill_key_groups(ctypes.byref(a))
+        self.key_groups = self._lib.ikl_paged_prefill_plan(ctypes.byref(a), max(self.ends), min(self.starts))
 
     def kernel_name(self) -> str:
         if self.path == "mfma_grouped":
@@ -999,7 +999,8 @@ class PreparedPagedPrefill:
             a.events[i] = events[i] if events is not None else None
         with torch.cuda.device(query.device):
             stream = torch.cuda.current_stream(query.device).cuda_stream
-            status = self._lib.ikl_paged_prefill_attention(ctypes.byref(a), ctypes.c_void_p(stream))
+            status = self._lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), self.key_groups,
+                                                                   ctypes.c_void_p(stream))
         _lib.check(status, "paged prefill attention")
         return out
 

@@ -1,7 +1,8 @@
 """The matrix-core prefill kernels at the edges of their plans, against the
 oracle: one, two and four waves per row (launches of up to 64, 256 and 512
-128-row workgroups, and two rounds behind long prefixes) and the kernel of
-launches past that. Key counts end on, before and after a 32-key tile and a
+128-row workgroups with long contexts, and two rounds behind long prefixes)
+and the kernel of launches past that or with short ones, and every plan on
+every shape. Key counts end on, before and after a 32-key tile and a
 group's last step, tables cross the kernels' 64-half windows, some entries
 lie outside the cache, rows end inside a 32-row group, one request has a
 single key and one pads most of its rows."""
@@ -20,7 +21,8 @@ pytestmark = pytest.mark.gpu
 
 # (expected groups, heads, kv heads, head dim, block size, starts, ends)
 PLANS = [
-    (4, 8, 2, 128, 16, [0, 0, 31, 95], [1, 33, 64, 129]),
+    (0, 8, 2, 128, 16, [0, 0, 31, 95], [1, 33, 64, 129]),
+    (4, 8, 2, 128, 16, [0, 0, 31, 255], [1, 33, 64, 289]),
     (4, 4, 1, 64, 32, [1500, 0], [1511, 97]),
     (4, 6, 2, 96, 48, [130, 40], [161, 60]),
     (4, 8, 8, 32, 16, [0, 160], [70, 193]),
@@ -29,10 +31,12 @@ PLANS = [
     (2, 24, 8, 96, 16, [0, 32, 64, 96, 128], [50, 64, 65, 97, 160]),
     (1, 32, 8, 128, 16, [0, 0, 31, 64, 1050], [225, 1, 64, 289, 1100]),
     (1, 32, 8, 64, 16, [0, 0, 31, 64, 0], [225, 1, 64, 289, 33]),
-    (1, 32, 8, 32, 32, [0] * 9, [250, 249, 33, 32, 31, 1, 250, 64, 65]),
+    (0, 32, 8, 32, 32, [0] * 9, [250, 249, 33, 32, 31, 1, 250, 64, 65]),
+    (1, 32, 8, 32, 32, [1000] + [0] * 8, [1250, 249, 33, 32, 31, 1, 250, 64, 65]),
     (1, 32, 4, 128, 16, [1200] * 17, [1325] + [1201 + 7 * i for i in range(16)]),  # two rounds, long prefixes
     (0, 32, 4, 128, 16, [0, 17] * 9, [128, 100, 1, 33, 32, 31, 127, 97, 96, 95, 65, 64, 63, 20, 50, 77, 128, 120]),
     (0, 32, 4, 64, 32, [0] * 18, [128, 100, 1, 33, 32, 31, 127, 97, 96, 95, 65, 64, 63, 20, 50, 77, 128, 120]),
+    (1, 32, 4, 96, 16, [1200] * 18, [1328] + [1201 + 7 * i for i in range(17)]),
     (0, 32, 4, 96, 16, [0] * 18, [128, 100, 1, 33, 32, 31, 127, 97, 96, 95, 65, 64, 63, 20, 50, 77, 128, 120]),
     (0, 32, 8, 64, 16, [400, 0, 500], [1100, 33, 601]),  # windows move
 ]
@@ -66,7 +70,7 @@ def test_plan_edges_over_the_fp8_cache(groups, heads, kv, dim, bs, starts, ends)
     q = randn_storage(torch.Generator().manual_seed(dim), (len(ends), heads, width, dim), act)
     prep = PreparedPagedPrefill(_device_fp8_cache(base, packed, act), base.device_tables(), starts, ends,
                                 num_heads=heads, query_width=width)
-    assert prep.key_groups == (1 if groups == 0 and dim == 96 else groups)
+    assert prep.key_groups == groups
     got = prep(storage_to_torch(q, act).cuda()).float().cpu().numpy()
     expected = po.paged_prefill_attention(po.to_f32(q, act), base.oracle_cache, base.tables, starts, ends)
     assert not np.isnan(got).any()
@@ -93,3 +97,38 @@ def test_entries_outside_the_cache(groups, heads, kv, starts, ends, dropped):
                                 query_width=q.shape[2])
     assert prep.key_groups == groups
     assert max_abs_err(prep(q), _expected_dropping_blocks(case, dropped)) < ATOL["bfloat16"]
+
+
+FORCED = [
+    (8, 2, 16, [0, 0, 31, 95], [1, 33, 64, 129]),
+    (6, 2, 48, [130, 40], [161, 60]),
+    (8, 8, 32, [0, 160, 3], [70, 193, 4]),
+    (8, 1, 16, [500, 0], [533, 64]),
+]
+
+
+@pytest.mark.parametrize("dim", [32, 64, 96, 128])
+@pytest.mark.parametrize("cache", ["same", "fp8"])
+@pytest.mark.parametrize("heads,kv,bs,starts,ends", FORCED)
+def test_every_plan_gives_the_same_result(heads, kv, bs, starts, ends, cache, dim):
+    from inferkernellab_amd import PreparedPagedPrefill
+
+    act = "bfloat16"
+    width = max(e - s for s, e in zip(starts, ends))
+    if cache == "fp8":
+        base, packed = _fp8_case(batch=len(ends), heads=heads, kv=kv, dim=dim, bs=bs, lengths=ends, act=act, seed=dim)
+        device = _device_fp8_cache(base, packed, act)
+        q = randn_storage(torch.Generator().manual_seed(dim), (len(ends), heads, width, dim), act)
+        expected = po.paged_prefill_attention(po.to_f32(q, act), base.oracle_cache, base.tables, starts, ends)
+        query, tables = storage_to_torch(q, act).cuda(), base.device_tables()
+    else:
+        case = make_prefill_case(starts=starts, ends=ends, num_heads=heads, num_kv_heads=kv, head_dim=dim,
+                                 block_size=bs, dtype=act, seed=heads + dim)
+        device, query, tables, expected = (case.base.device_cache(), case.device_query(), case.base.device_tables(),
+                                           case.expected())
+    prep = PreparedPagedPrefill(device, tables, starts, ends, num_heads=heads, query_width=width)
+    for plan in (0, 1, 2, 4):
+        prep.key_groups = plan
+        got = prep(query, out=torch.full_like(query, float("nan"))).float().cpu().numpy()
+        assert not np.isnan(got).any()
+        assert max_abs_err(got, expected, act) < ATOL[act], plan

@@ -1,0 +1,84 @@
+"""The rule that splits a prefill launch's keys between waves: the lines it
+draws, that it goes by the ranges of the requests and not by how wide a table
+the caller keeps, and what it answers and refuses. Runs on the CPU."""
+
+import ctypes
+
+import pytest
+
+from inferkernellab_amd import _lib
+
+
+def _args(batch, heads, kv, dim, width, table_blocks, dtype=_lib.IKL_BF16, cache=0, **kw):
+    a = _lib.PagedPrefillArgs()
+    a.batch, a.query_width, a.num_heads, a.num_kv_heads = batch, width, heads, kv
+    a.head_dim, a.block_size, a.dtype, a.cache_dtype, a.path = dim, 16, dtype, cache, -1
+    a.table_width, a.num_blocks = table_blocks, 1 << 20
+    for name, value in kw.items():
+        setattr(a, name, value)
+    return a
+
+
+def _plan(a, longest, start):
+    return _lib.load().ikl_paged_prefill_plan(ctypes.byref(a), longest, start)
+
+
+@pytest.mark.parametrize("batch,heads,kv,dim,width", [(8, 32, 8, 128, 512), (4, 32, 8, 128, 1024), (6, 32, 8, 128, 512),
+                                                      (8, 32, 8, 64, 512), (4, 32, 8, 96, 1024)])
+def test_a_wide_table_changes_no_plan(batch, heads, kv, dim, width):
+    tight, wide = (_args(batch, heads, kv, dim, width, n) for n in (width // 16, 8192 // 16))
+    lib = _lib.load()
+    assert lib.ikl_paged_prefill_key_groups(ctypes.byref(wide)) == lib.ikl_paged_prefill_key_groups(ctypes.byref(tight))
+    assert _plan(wide, width, 0) == _plan(tight, width, 0) == 0
+
+
+FP8 = _lib.IKL_FP8_E4M3
+# (batch, heads, kv heads, dim, cache, start, tokens, plan): the short side of
+# each line, where splitting was measured slower, and the long side
+LINES = [
+    (4, 32, 8, 128, 0, 0, 64, 0), (2, 32, 8, 128, 0, 120, 8, 0), (1, 32, 32, 128, 0, 0, 96, 0),
+    (8, 32, 8, 64, 0, 0, 64, 0), (2, 32, 8, 64, 0, 120, 8, 4), (8, 32, 8, 128, 0, 480, 32, 4),
+    (1, 8, 2, 128, 0, 0, 256, 4), (1, 32, 32, 128, 0, 0, 192, 2),
+    (8, 32, 8, 128, 0, 0, 128, 0), (8, 32, 8, 128, FP8, 0, 128, 0), (32, 32, 8, 128, 0, 480, 32, 0),
+    (16, 32, 8, 64, 0, 0, 64, 0), (8, 8, 2, 128, 0, 0, 256, 2), (1, 32, 8, 128, 0, 0, 1024, 2),
+    (8, 32, 32, 128, 0, 0, 256, 0), (64, 32, 8, 128, 0, 480, 32, 0), (16, 32, 32, 64, 0, 0, 128, 0),
+    (2, 32, 8, 128, 0, 0, 1024, 1), (8, 16, 4, 128, 0, 0, 512, 1),
+    (25, 32, 8, 128, 0, 128, 128, 0), (4, 32, 8, 128, 0, 2048, 1024, 0), (3, 32, 8, 64, 0, 1024, 1024, 0),
+    (3, 32, 8, 128, 0, 2048, 1024, 1), (4, 32, 8, 128, FP8, 2048, 1024, 1), (4, 32, 8, 64, 0, 2048, 1024, 1),
+    (4, 32, 8, 96, 0, 2048, 1024, 1), (62, 32, 1, 128, 0, 64, 64, 0),
+    (16, 32, 32, 96, FP8, 0, 128, 0), (64, 32, 32, 32, FP8, 0, 64, 0), (4, 32, 8, 32, 0, 0, 2048, 1),
+    (8, 32, 8, 96, FP8, 0, 4096, 1), (8, 32, 8, 96, 0, 0, 4096, 0), (8, 32, 8, 128, 0, 0, 4096, 0),
+]
+
+
+@pytest.mark.parametrize("batch,heads,kv,dim,cache,start,tokens,plan", LINES)
+def test_lines_of_the_rule(batch, heads, kv, dim, cache, start, tokens, plan):
+    a = _args(batch, heads, kv, dim, tokens, 4096, cache=cache)
+    assert _plan(a, start + tokens, start) == plan
+
+
+def test_unknown_ranges_count_as_the_query_width_from_position_0():
+    for width in (8, 64, 300, 512, 2048):
+        a = _args(2, 32, 8, 128, width, 512)
+        assert _plan(a, 0, 0) == _plan(a, width, 0) == _lib.load().ikl_paged_prefill_key_groups(ctypes.byref(a))
+
+
+def test_the_other_path_has_one_plan_and_takes_no_other():
+    lib = _lib.load()
+    ptr = ctypes.addressof(ctypes.create_string_buffer(64)) & ~15
+    a = _args(4, 32, 8, 64, 1024, 64, dtype=_lib.IKL_F32)
+    assert _plan(a, 1024, 0) == 0
+    for name in ("query", "k_cache", "v_cache", "block_tables", "query_starts", "context_lens", "out"):
+        setattr(a, name, ptr)
+    for plan in (1, 2, 4):
+        assert lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), plan, None) == _lib.IKL_EINVAL
+    a.dtype = _lib.IKL_BF16
+    for plan in (-2, 3, 5, 8):
+        assert lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), plan, None) == _lib.IKL_EINVAL
+    assert b"plan" in lib.ikl_last_error()
+
+
+def test_invalid_ranges_are_refused():
+    a = _args(1, 8, 2, 64, 16, 8)
+    assert _plan(a, -1, 0) == _lib.IKL_EINVAL and _plan(a, 16, -1) == _lib.IKL_EINVAL
+    assert _lib.load().ikl_paged_prefill_plan(None, 0, 0) == _lib.IKL_EINVAL
