@@ -393,10 +393,25 @@ __global__ __launch_bounds__(64 * FWAVES, f32_waves(DP)) void paged_prefill_f32_
     }
   } else {
     // padding row: the value at position 0 (zero when its block is masked),
-    // in 4-byte words; the row's four lanes take every fourth
+    // the row's four lanes taking every fourth quad, or word
     const int ph = end > 0 ? pf_block(p, b, 0) : -1;
-    const uint32_t *src = ph >= 0 ? reinterpret_cast<const uint32_t *>(vbase + ph * p.v_sb * EB) : nullptr;
-    for (int i = grp; i < D * EB / 4; i += 4) reinterpret_cast<uint32_t *>(dst)[i] = src ? src[i] : 0u;
+    const char *src = ph >= 0 ? vbase + ph * p.v_sb * EB : nullptr;
+    if (vec) {
+      typename Q4::raw w[DP / 16];
+#pragma unroll
+      for (int i = 0; i < DP / 16; ++i) {
+        const int d = 16 * i + 4 * grp;
+        w[i] = src && d < D ? Q4::load(src + d * EB) : Q4::zero();
+      }
+#pragma unroll
+      for (int i = 0; i < DP / 16; ++i) {
+        const int d = 16 * i + 4 * grp;
+        if (d < D) *reinterpret_cast<typename Q4::raw *>(dst + d * EB) = w[i];
+      }
+    } else {
+      for (int i = grp; i < D * EB / 4; i += 4)
+        reinterpret_cast<uint32_t *>(dst)[i] = src ? reinterpret_cast<const uint32_t *>(src)[i] : 0u;
+    }
   }
 }
 
