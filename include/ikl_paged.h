@@ -269,19 +269,22 @@ int ikl_paged_prefill_attention(const ikl_paged_prefill_args *args, void *stream
 
 /* How a prefill launch runs. On the matrix-core path: 1, 2 or 4 waves share
  * each row (launches that leave the chip idle), 0 when all waves of a
- * workgroup walk the keys together; 0 on the other path. longest_context /
+ * workgroup walk the keys together. On the other path: IKL_PREFILL_ROWS for
+ * one wave per row (short contexts, wide rows), 0 for the fp32 matrix cores.
+ * longest_context /
  * shortest_start: the largest element of context_lens and the smallest of
  * query_starts where the host knows them, else 0. Planning only: tensors are
- * not looked at, every plan gives the same result, and a plan serves every
- * launch of the same sizes. Negative on invalid sizes. */
+ * not looked at, every plan of the path gives the same result, and a plan
+ * serves every launch of the same sizes. Negative on invalid sizes. */
 #define IKL_PREFILL_AUTO (-1)
+#define IKL_PREFILL_ROWS 8
 int32_t ikl_paged_prefill_plan(const ikl_paged_prefill_args *args, int64_t longest_context, int64_t shortest_start);
 
 /* ikl_paged_prefill_attention with a plan of ikl_paged_prefill_plan;
  * IKL_PREFILL_AUTO = the plan of unknown ranges, which that entry runs with. */
 int ikl_paged_prefill_attention_planned(const ikl_paged_prefill_args *args, int32_t plan, void *stream);
 
-/* ikl_paged_prefill_plan of unknown ranges. */
+/* ikl_paged_prefill_plan of unknown ranges; 0 off the matrix-core path. */
 int32_t ikl_paged_prefill_key_groups(const ikl_paged_prefill_args *args);
 
 /* Kernel family a prefill launch uses: IKL_PATH_MFMA_GROUPED for fp16/bf16

@@ -22,6 +22,7 @@ IKL_F16, IKL_BF16, IKL_F32, IKL_FP8_E4M3 = 0, 1, 2, 3
 IKL_I32, IKL_I64 = 0, 1
 IKL_OK, IKL_EINVAL, IKL_EUNSUPPORTED, IKL_ELAUNCH, IKL_EWORKSPACE = 0, -1, -2, -3, -4
 IKL_PATH_MHA_FALLBACK, IKL_PATH_SCALAR_GROUPED, IKL_PATH_MFMA_GROUPED = 0, 1, 2
+IKL_PREFILL_AUTO, IKL_PREFILL_ROWS = -1, 8  # plans of ikl_paged_prefill_plan
 # findings of ikl_check_metadata
 IKL_CHECK_LENGTH_POSITIVE, IKL_CHECK_LENGTH_CAPACITY, IKL_CHECK_BLOCK_ID, IKL_CHECK_LENGTH_MAX = 1, 2, 4, 8
 # IKL_ABI_VERSION of the header these mirrors follow; load() refuses a

@@ -30,12 +30,16 @@
 //    ds_read_b64_tr_b16 of the staged tile.
 //
 //  * every other dtype / head_dim / block size: paged_prefill_f32_kernel
-//    (paged_prefill_f32.hip, fp32 matrix cores) up to head_dim 256; wider
+//    (paged_prefill_f32.hip, fp32 matrix cores) up to head_dim 256; launches
+//    with short contexts or few rows per KV head (prefill_by_rows) and wider
 //    16-bit rows run paged_prefill_scalar_kernel, one wave per (request,
 //    head, row), keys in sequence, fp32 online softmax.
 //
 // Blocks whose table entry lies outside [0, num_blocks) are masked as in the
 // decode kernels; no load ever leaves the cache.
+#include <algorithm>
+#include <cmath>
+
 #include "ikl_common.h"
 #include "mfma_ops.h"
 #include "paged_attn.h"
@@ -462,10 +466,16 @@ __global__ __launch_bounds__(64 * PWAVES) IKL_PREFILL_WAVES_ATTR void paged_pref
 
 // ------------------------------------------------------------------ VALU
 // One wave per (request, head, row). The lanes split the row's head_dim in
-// 4-byte granules (two 16-bit elements; up to 4 per lane), walk
+// 4-byte granules (one fp32 or two 16-bit elements; up to 4 per lane), walk
 // the keys in order and keep an fp32 online softmax in the log2 domain.
 template <typename Tag>
 struct granule;
+template <>
+struct granule<f32_tag> {
+  static constexpr int EB = 4, PER = 1;
+  __device__ static inline void unpack(uint32_t w, float *x) { x[0] = __uint_as_float(w); }
+  __device__ static inline uint32_t pack(const float *x) { return __float_as_uint(x[0]); }
+};
 template <>
 struct granule<bf16_tag> {
   static constexpr int EB = 2, PER = 2;
@@ -644,14 +654,46 @@ int64_t prefill_row_blocks(const ikl_paged_prefill_args *a) {
 
 int64_t prefill_bh_pad(const ikl_paged_prefill_args *a) { return (a->batch * a->num_kv_heads + 7) / 8 * 8; }
 
-// The plan of a launch of the matrix-core family. A caller that does not know
-// its ranges (0) most likely has a request that fills the query width, so its
-// longest context is taken to be that, from position 0.
-int prefill_plan(const ikl_paged_prefill_args *a, int64_t longest_context, int64_t shortest_start) {
+// Whether a launch off the 16-bit matrix cores runs one wave per row. The fp32
+// matrix-core kernel works on 64-row workgroups and 32-key tiles: of few keys
+// or few rows it computes mostly padding. us, fp32 kernel / one wave per row
+// (fp32, 32/32 heads, requests x keys before + tokens):
+//   64 dims: 64 x (0 + 1) 19.6 / 4.0   4 x 2-5 tokens 8.6 / 4.3
+//            4 x 8-17 tokens 7.9 / 8.9   4 x (255 + 1) 20.4 / 117
+//   256 dims: 64 x (0 + 1) 82 / 4.2   64 x (2047 + 1) 3311 / 2241
+//            16 x (2047 + 1) 829 / 1719   4 x 16-33 tokens 16 / 26
+// So both times are estimated from what bounds them and compared. One wave
+// per row: the dependent walk along the longest context, 0.45 us a key, and
+// the keys of all rows, 0.073 ns each and 0.08 ns per KB of their rows. The
+// fp32 kernel: as many rounds of resident workgroups as the launch has, each
+// with a start and a time per tile by the compiled width. Fitted to 3900
+// launches around the line (18 % scatter for one wave per row, 10-15 % for
+// the other). With a seventh in favour of one wave per row, 6 of them are
+// more than 3 % slower than that kernel and one more than 10 %; choosing by
+// hindsight would be 1.4 % faster on the average.
+bool prefill_by_rows(const ikl_paged_prefill_args *a, int64_t longest) {
+  if (a->head_dim > PREFILL_F32_MAX_DIM) return true;
+  const int w = a->head_dim <= 32 ? 0 : a->head_dim <= 64 ? 1 : a->head_dim <= 96 ? 2 : a->head_dim <= 128 ? 3 : 4;
+  constexpr double resident[] = {768, 768, 512, 512, 256}, start[] = {3.5, 5.0, 6.5, 8.0, 8.0},
+                   tile[] = {1.5, 2.2, 2.8, 3.7, 6.0};  // workgroups, us, us
+  const double rows = (double)a->query_width * (a->num_heads / a->num_kv_heads);
+  const double workgroups = std::ceil(rows / 64) * (double)prefill_bh_pad(a);
+  const double f32 = std::ceil(workgroups / resident[w]) * (start[w] + tile[w] * std::ceil((double)longest / 32));
+  const double mean = std::max(1.0, (double)longest - 0.5 * (double)(a->query_width - 1));
+  const double waves = (double)a->batch * a->num_heads * (double)a->query_width;
+  const double row_bytes = a->head_dim * (a->dtype == IKL_F32 ? 4.0 : 2.0);
+  return 2.6 + 0.45 * (double)longest + (7.3e-5 + 8e-8 * row_bytes) * waves * mean <= 1.15 * f32;
+}
+
+// The plan of a launch. A caller that does not know its ranges (0) most
+// likely has a request that fills the query width, so its longest context is
+// taken to be that, from position 0.
+int prefill_plan(const ikl_paged_prefill_args *a, int path, int64_t longest_context, int64_t shortest_start) {
+  const int64_t longest = longest_context > 0 ? longest_context : a->query_width;
+  if (path != IKL_PATH_MFMA_GROUPED) return prefill_by_rows(a, longest) ? IKL_PREFILL_ROWS : 0;
   const int64_t row_blocks = prefill_row_blocks(a);
-  return prefill_key_groups(row_blocks * prefill_bh_pad(a), row_blocks,
-                            longest_context > 0 ? longest_context : a->query_width,
-                            shortest_start >= a->query_width, a->head_dim, a->cache_dtype == IKL_FP8_E4M3);
+  return prefill_key_groups(row_blocks * prefill_bh_pad(a), row_blocks, longest, shortest_start >= a->query_width,
+                            a->head_dim, a->cache_dtype == IKL_FP8_E4M3);
 }
 
 bool aligned(const void *ptr, int64_t bytes) { return ((uintptr_t)ptr) % bytes == 0; }
@@ -670,12 +712,14 @@ extern "C" int32_t ikl_paged_prefill_plan(const ikl_paged_prefill_args *a, int64
   if (!a || a->batch <= 0 || a->query_width <= 0 || a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0 ||
       longest_context < 0 || shortest_start < 0)
     return fail(IKL_EINVAL, "ikl_paged_prefill_plan: invalid arguments");
-  if (!prefill_mfma_supported(a->dtype, a->head_dim, a->block_size) || a->path == IKL_PATH_SCALAR_GROUPED) return 0;
-  return prefill_plan(a, longest_context, shortest_start);
+  const int path = a->path == IKL_PATH_SCALAR_GROUPED ? a->path
+                                                      : ikl_paged_prefill_path(a->dtype, a->head_dim, a->block_size);
+  return prefill_plan(a, path, longest_context, shortest_start);
 }
 
 extern "C" int32_t ikl_paged_prefill_key_groups(const ikl_paged_prefill_args *a) {
-  return ikl_paged_prefill_plan(a, 0, 0);
+  const int32_t plan = ikl_paged_prefill_plan(a, 0, 0);
+  return plan == IKL_PREFILL_ROWS ? 0 : plan;
 }
 
 extern "C" int ikl_paged_prefill_attention(const ikl_paged_prefill_args *args, void *stream) {
@@ -714,9 +758,9 @@ extern "C" int ikl_paged_prefill_attention_planned(const ikl_paged_prefill_args 
   const int ceb = kv8 ? 1 : eb;  // cache bytes per element
   if (path != IKL_PATH_MFMA_GROUPED && path != IKL_PATH_SCALAR_GROUPED)
     return fail(IKL_EINVAL, "ikl_paged_prefill_attention: path must be -1, IKL_PATH_SCALAR_GROUPED or IKL_PATH_MFMA_GROUPED");
-  if (plan != IKL_PREFILL_AUTO && plan != 0 &&
-      (path != IKL_PATH_MFMA_GROUPED || (plan != 1 && plan != 2 && plan != 4)))
-    return fail(IKL_EINVAL, "ikl_paged_prefill_attention: plan must be -1, 0 or, on the matrix-core path, 1, 2 or 4");
+  const bool split = plan == 1 || plan == 2 || plan == 4;
+  if (plan != IKL_PREFILL_AUTO && plan != 0 && !(path == IKL_PATH_MFMA_GROUPED ? split : plan == IKL_PREFILL_ROWS))
+    return fail(IKL_EINVAL, "ikl_paged_prefill_attention: plan must be IKL_PREFILL_AUTO, 0 or one of the path's own");
   if (path == IKL_PATH_MFMA_GROUPED && auto_path != IKL_PATH_MFMA_GROUPED)
     return fail(IKL_EUNSUPPORTED, "ikl_paged_prefill_attention: no MFMA kernel for this dtype / head_dim / block_size");
   if (path == IKL_PATH_MFMA_GROUPED) {
@@ -791,6 +835,7 @@ extern "C" int ikl_paged_prefill_attention_planned(const ikl_paged_prefill_args 
   hipEvent_t ev0 = static_cast<hipEvent_t>(a->events[0]), ev1 = static_cast<hipEvent_t>(a->events[1]);
   if (ev0 && hipEventRecord(ev0, s) != hipSuccess) return check_launch("ikl_paged_prefill_attention: event record");
   hipError_t err;
+  if (plan == IKL_PREFILL_AUTO) plan = prefill_plan(a, path, 0, 0);
   if (path == IKL_PATH_MFMA_GROUPED) {
     constexpr int NG = PREFILL_NG;
     p.bh_pad = prefill_bh_pad(a);
@@ -804,7 +849,6 @@ extern "C" int ikl_paged_prefill_attention_planned(const ikl_paged_prefill_args 
     p.stream_major = p.row_blocks >= 64 && !p.kv_fp8;
     if (blocks > 0x7fffffffLL) return fail(IKL_EINVAL, "ikl_paged_prefill_attention: launch too large");
     const dim3 grid((unsigned)blocks);
-    if (plan == IKL_PREFILL_AUTO) plan = prefill_plan(a, 0, 0);
     if (plan > 0)
       err = launch_prefill_split(p, a->dtype, plan, s);
     else if (a->dtype == IKL_BF16)
@@ -816,15 +860,16 @@ extern "C" int ikl_paged_prefill_attention_planned(const ikl_paged_prefill_args 
   } else {
     const int64_t blocks = a->batch * a->num_heads * a->query_width;
     if (blocks > 0x7fffffffLL) return fail(IKL_EINVAL, "ikl_paged_prefill_attention: launch too large");
-    // The fp32 matrix cores wherever their kernel is compiled; 16-bit rows
-    // of 257-512 elements (fp32 rows end at 256) keep one wave per row: a
-    // 512-wide accumulator and its query would fill a wave's registers.
-    if (a->head_dim <= PREFILL_F32_MAX_DIM) {
+    // 16-bit rows of 257-512 elements (fp32 rows end at 256) always run one
+    // wave per row: a 512-wide accumulator and its query would fill a wave's
+    // registers.
+    if (plan != IKL_PREFILL_ROWS && a->head_dim <= PREFILL_F32_MAX_DIM) {
       err = launch_prefill_f32(p, a->dtype, s);
     } else {
       const dim3 grid((unsigned)blocks);
       if (a->dtype == IKL_BF16) paged_prefill_scalar_kernel<bf16_tag><<<grid, 64, 0, s>>>(p);
-      else paged_prefill_scalar_kernel<f16_tag><<<grid, 64, 0, s>>>(p);
+      else if (a->dtype == IKL_F16) paged_prefill_scalar_kernel<f16_tag><<<grid, 64, 0, s>>>(p);
+      else paged_prefill_scalar_kernel<f32_tag><<<grid, 64, 0, s>>>(p);
       err = hipGetLastError();
     }
   }

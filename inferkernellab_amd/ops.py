@@ -959,12 +959,17 @@ class PreparedPagedPrefill:
         a.scale = float(scale if scale is not None else layout.head_dim**-0.5)
         a.path = _PATH_IDS[self.path]
         self._args = a
-        self.key_groups = self._lib.ikl_paged_prefill_plan(ctypes.byref(a), max(self.ends), min(self.starts))
+        self.plan = self._lib.ikl_paged_prefill_plan(ctypes.byref(a), max(self.ends), min(self.starts))
+
+    @property
+    def key_groups(self) -> int:
+        """Waves that share a row on the matrix-core path, else 0."""
+        return self.plan if self.path == "mfma_grouped" else 0
 
     def kernel_name(self) -> str:
         if self.path == "mfma_grouped":
-            return "paged_prefill_split_kernel" if self.key_groups else "paged_prefill_mfma_kernel"
-        return "paged_prefill_f32_kernel" if self.shape[-1] <= 256 else "paged_prefill_scalar_kernel"
+            return "paged_prefill_split_kernel" if self.plan else "paged_prefill_mfma_kernel"
+        return "paged_prefill_scalar_kernel" if self.plan == _lib.IKL_PREFILL_ROWS else "paged_prefill_f32_kernel"
 
     def __call__(self, query: torch.Tensor, layer: int = 0, *, out: torch.Tensor | None = None,
                  events=None) -> torch.Tensor:
@@ -999,7 +1004,7 @@ class PreparedPagedPrefill:
             a.events[i] = events[i] if events is not None else None
         with torch.cuda.device(query.device):
             stream = torch.cuda.current_stream(query.device).cuda_stream
-            status = self._lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), self.key_groups,
+            status = self._lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), self.plan,
                                                                    ctypes.c_void_p(stream))
         _lib.check(status, "paged prefill attention")
         return out

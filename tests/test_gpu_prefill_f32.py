@@ -14,16 +14,17 @@ from tests.helpers import ATOL, make_prefill_case, max_abs_err
 pytestmark = pytest.mark.gpu
 
 
-def _prepare(case, query):
+def _prepare(case, query, plan=0):
     from inferkernellab_amd import PreparedPagedPrefill
 
     prep = PreparedPagedPrefill(case.base.device_cache(), case.base.device_tables(), case.starts, case.ends,
                                 num_heads=query.shape[1], query_width=query.shape[2], path="scalar_grouped")
-    assert prep.kernel_name() == "paged_prefill_f32_kernel"
+    prep.plan = plan  # whichever the rule takes for these sizes
+    assert prep.kernel_name() == ("paged_prefill_scalar_kernel" if plan else "paged_prefill_f32_kernel")
     return prep
 
 
-@pytest.mark.parametrize("heads,kv,dim,bs,dtype,starts,ends", [
+EDGES = [
     (4, 4, 8, 4, "float32", [0, 0, 0], [31, 32, 33]),
     (6, 2, 20, 5, "float32", [0, 64], [65, 97]),
     (6, 2, 33, 16, "float32", [7, 31], [40, 33]),  # odd rows: never aligned to four
@@ -37,12 +38,16 @@ def _prepare(case, query):
     (8, 2, 80, 16, "bfloat16", [0, 40], [90, 75]),
     (4, 2, 34, 16, "float16", [0], [50]),  # 4-byte rows
     (4, 1, 128, 8, "float16", [16, 0], [81, 64]),
-])
-def test_tile_edges(heads, kv, dim, bs, dtype, starts, ends):
+]
+
+
+@pytest.mark.parametrize("plan", [0, 8])  # fp32 matrix cores, one wave per row
+@pytest.mark.parametrize("heads,kv,dim,bs,dtype,starts,ends", EDGES)
+def test_tile_edges(heads, kv, dim, bs, dtype, starts, ends, plan):
     case = make_prefill_case(starts=starts, ends=ends, num_heads=heads, num_kv_heads=kv, head_dim=dim, block_size=bs,
                              dtype=dtype, seed=heads + dim + bs, table_slack=1)
     q = case.device_query()
-    got = _prepare(case, q)(q)
+    got = _prepare(case, q, plan)(q)
     # fp32: a few ulp per product over <= 257 keys; 16-bit: the output's rounding
     assert max_abs_err(got, case.expected()) <= (1e-5 if dtype == "float32" else ATOL[dtype])
 

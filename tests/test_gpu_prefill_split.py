@@ -128,7 +128,7 @@ def test_every_plan_gives_the_same_result(heads, kv, bs, starts, ends, cache, di
                                            case.expected())
     prep = PreparedPagedPrefill(device, tables, starts, ends, num_heads=heads, query_width=width)
     for plan in (0, 1, 2, 4):
-        prep.key_groups = plan
+        prep.plan = plan
         got = prep(query, out=torch.full_like(query, float("nan"))).float().cpu().numpy()
         assert not np.isnan(got).any()
         assert max_abs_err(got, expected, act) < ATOL[act], plan

@@ -1,6 +1,7 @@
-"""The rule that splits a prefill launch's keys between waves: the lines it
-draws, that it goes by the ranges of the requests and not by how wide a table
-the caller keeps, and what it answers and refuses. Runs on the CPU."""
+"""The rules that plan a prefill launch (keys split between waves on the 16-bit
+matrix cores; fp32 matrix cores or one wave per row elsewhere): the lines they
+draw, that they go by the ranges of the requests and not by how wide a table
+the caller keeps, and what they answer and refuse. Runs on the CPU."""
 
 import ctypes
 
@@ -63,17 +64,38 @@ def test_unknown_ranges_count_as_the_query_width_from_position_0():
         assert _plan(a, 0, 0) == _plan(a, width, 0) == _lib.load().ikl_paged_prefill_key_groups(ctypes.byref(a))
 
 
-def test_the_other_path_has_one_plan_and_takes_no_other():
+ROWS = _lib.IKL_PREFILL_ROWS
+# (batch, heads, kv heads, dim, dtype, start, tokens, plan), off the 16-bit
+# matrix cores: one wave per row where it was measured the faster
+OTHER_LINES = [
+    (64, 32, 32, 64, _lib.IKL_F32, 0, 1, ROWS), (4, 32, 8, 64, _lib.IKL_F32, 0, 5, ROWS),
+    (1, 32, 8, 256, _lib.IKL_F32, 0, 12, ROWS), (64, 32, 32, 256, _lib.IKL_F32, 2047, 1, ROWS),
+    (64, 32, 32, 256, _lib.IKL_BF16, 255, 1, ROWS), (64, 8, 1, 80, _lib.IKL_BF16, 0, 5, ROWS),
+    (1, 8, 2, 512, _lib.IKL_BF16, 0, 4096, ROWS),  # no wider kernel
+    (4, 32, 8, 64, _lib.IKL_F32, 255, 1, 0), (16, 32, 32, 256, _lib.IKL_F32, 2047, 1, 0),
+    (64, 32, 32, 128, _lib.IKL_F32, 255, 1, 0), (4, 32, 8, 64, _lib.IKL_F32, 0, 64, 0),
+    (4, 32, 8, 64, _lib.IKL_F32, 0, 512, 0), (1, 8, 1, 80, _lib.IKL_BF16, 0, 33, 0),
+    (64, 32, 8, 32, _lib.IKL_F32, 0, 17, 0),
+]
+
+
+@pytest.mark.parametrize("batch,heads,kv,dim,dtype,start,tokens,plan", OTHER_LINES)
+def test_lines_between_the_fp32_matrix_cores_and_one_wave_per_row(batch, heads, kv, dim, dtype, start, tokens, plan):
+    a = _args(batch, heads, kv, dim, tokens, 4096, dtype=dtype, path=_lib.IKL_PATH_SCALAR_GROUPED)
+    assert _plan(a, start + tokens, start) == plan
+    assert _lib.load().ikl_paged_prefill_key_groups(ctypes.byref(a)) == 0
+
+
+def test_a_plan_of_the_other_path_is_refused():
     lib = _lib.load()
     ptr = ctypes.addressof(ctypes.create_string_buffer(64)) & ~15
     a = _args(4, 32, 8, 64, 1024, 64, dtype=_lib.IKL_F32)
-    assert _plan(a, 1024, 0) == 0
     for name in ("query", "k_cache", "v_cache", "block_tables", "query_starts", "context_lens", "out"):
         setattr(a, name, ptr)
     for plan in (1, 2, 4):
         assert lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), plan, None) == _lib.IKL_EINVAL
     a.dtype = _lib.IKL_BF16
-    for plan in (-2, 3, 5, 8):
+    for plan in (-2, 3, 5, ROWS):
         assert lib.ikl_paged_prefill_attention_planned(ctypes.byref(a), plan, None) == _lib.IKL_EINVAL
     assert b"plan" in lib.ikl_last_error()
 
