@@ -616,6 +616,7 @@ bool prefill_mfma_supported(int dtype, int head_dim, int block_size) {
 //   one resident round: 2 x 1024              36.6 / 32.8 / 38.3 / -
 //     but 8 x 128-256, 32/32 heads            19.9 / 20.7 / 25.8 / -
 //     64 x (480 + 32)                         39.4 / 43.0 / 59.4 / -
+//     32 x (1984 + 64)                        93.7 / 97.7 / -
 // Up to 96 dims a step costs less against the rest of the launch and the
 // lines lie lower. Chunks behind prefixes of at least their width (`even`)
 // have rows of nearly one length, and the whole chip walks keys to the end:
@@ -639,7 +640,8 @@ int prefill_key_groups(int64_t blocks, int64_t row_blocks, int64_t longest, bool
   if (blocks <= 64 && longest >= (narrow ? 128 : 256)) return 4;
   if (blocks <= 128 && longest >= (narrow ? 160 : 192)) return 2;
   if (blocks <= 256 && longest >= (even ? 1024 : 320)) return 2;
-  if (blocks <= 512) return longest >= (even ? 1024 : head_dim <= 64 ? 257 : 512) ? 1 : 0;
+  if (blocks <= 512 && even) return longest >= 1024 && (narrow || row_blocks >= 3) ? 1 : 0;
+  if (blocks <= 512) return longest >= (head_dim <= 64 ? 257 : 512) ? 1 : 0;
   if (longest < 1024 || row_blocks < 2) return 0;
   if (head_dim == 32 || (head_dim == 96 && kv8)) return 1;
   if (blocks > 1024 || row_blocks < 3 || !even) return 0;

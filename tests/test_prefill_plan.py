@@ -43,6 +43,7 @@ LINES = [
     (8, 32, 8, 128, 0, 0, 128, 0), (8, 32, 8, 128, FP8, 0, 128, 0), (32, 32, 8, 128, 0, 480, 32, 0),
     (16, 32, 8, 64, 0, 0, 64, 0), (8, 8, 2, 128, 0, 0, 256, 2), (1, 32, 8, 128, 0, 0, 1024, 2),
     (8, 32, 32, 128, 0, 0, 256, 0), (64, 32, 8, 128, 0, 480, 32, 0), (16, 32, 32, 64, 0, 0, 128, 0),
+    (32, 32, 8, 128, 0, 1984, 64, 0), (32, 32, 8, 96, 0, 1984, 64, 1), (2, 32, 8, 128, 0, 2048, 1024, 1),
     (2, 32, 8, 128, 0, 0, 1024, 1), (8, 16, 4, 128, 0, 0, 512, 1),
     (25, 32, 8, 128, 0, 128, 128, 0), (4, 32, 8, 128, 0, 2048, 1024, 0), (3, 32, 8, 64, 0, 1024, 1024, 0),
     (3, 32, 8, 128, 0, 2048, 1024, 1), (4, 32, 8, 128, FP8, 2048, 1024, 1), (4, 32, 8, 64, 0, 2048, 1024, 1),
