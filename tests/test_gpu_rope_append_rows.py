@@ -28,6 +28,19 @@ def _rotate(x, cos, sin):
     (torch.bfloat16, 128, 32, 32, 3),
     (torch.bfloat16, 128, 32, 8, 1025),
     (torch.float16, 64, 0, 2, 20),
+    # past the bounds (512 rows up to 64 dims, 1024 past that) up to which an
+    # FP8 row has a workgroup of its own, and four rows a token
+    (torch.bfloat16, 16, 3, 1, 110),
+    (torch.bfloat16, 64, 4, 2, 64),
+    (torch.bfloat16, 64, 4, 2, 65),
+    (torch.bfloat16, 80, 4, 2, 130),
+    (torch.float16, 144, 6, 3, 90),
+    (torch.bfloat16, 272, 3, 1, 210),
+    (torch.bfloat16, 512, 2, 2, 172),
+    (torch.float32, 48, 2, 2, 90),
+    (torch.float16, 128, 2, 1, 700),
+    (torch.bfloat16, 128, 8, 2, 85),
+    (torch.bfloat16, 128, 8, 2, 86),
 ])
 def test_rows_and_groups(dtype, dim, heads, kv, tokens, fp8):
     from inferkernellab_amd import ops
