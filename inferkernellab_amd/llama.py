@@ -22,6 +22,7 @@ to the activation dtype) for seeded random-weight models.
 from __future__ import annotations
 
 import math
+import sys
 import time
 from dataclasses import dataclass
 from typing import Any, Sequence
@@ -151,6 +152,13 @@ def random_llama(config: LlamaConfig, *, seed: int = 0, device="cuda",
 
 
 # --------------------------------------------------------------- the runner
+def _plain_row_norm(norm) -> bool:
+    """True when calling `norm` normalises each row by itself and nothing else
+    sees the call: RMSNorm here, or Transformers' where that is loaded."""
+    hf = getattr(sys.modules.get("transformers.models.llama.modeling_llama"), "LlamaRMSNorm", RMSNorm)
+    return layer_ops.plain_module(norm, RMSNorm) or layer_ops.plain_module(norm, hf)
+
+
 CAPTURE_FREE = 4 << 30  # device memory that a step's capture is sure to fit in
 
 
@@ -494,11 +502,16 @@ class LlamaPagedDecodeRunner:
             hidden, x = self._add_norm(layer.post_attention_layernorm, hidden,
                                        att.o_proj(o.reshape(b, t, self.num_heads * self.head_dim)))
             delta = self._mlp(layer.mlp, x)
-        # Only the chunks' last rows are read. Where a module between them
-        # and the logits is hooked or not a plain one, it sees all rows.
-        last = torch.tensor([n - 1 for n in spans], device=self.device)
-        rows = torch.arange(b, device=self.device)
-        if layer_ops.unhooked(m.norm) and layer_ops.plain_module(self.model.lm_head, nn.Linear):
+        return self._last_logits(hidden, delta, spans)
+
+    def _last_logits(self, hidden: torch.Tensor, delta: torch.Tensor | None, spans) -> torch.Tensor:
+        """Logits [B, vocab] of the last row of each chunk of hidden (+ delta)
+        [B, T, hidden]. Where the final norm or the head is hooked or not one
+        known to work row by row, it sees all rows."""
+        m = self.model.model
+        last = torch.tensor([n - 1 for n in spans], device=hidden.device)
+        rows = torch.arange(len(spans), device=hidden.device)
+        if _plain_row_norm(m.norm) and layer_ops.plain_module(self.model.lm_head, nn.Linear):
             hidden = hidden[rows, last]
             delta = None if delta is None else delta[rows, last]
             return self.model.lm_head(self._add_norm(m.norm, hidden, delta)[1])
