@@ -21,6 +21,7 @@ to the activation dtype) for seeded random-weight models.
 
 from __future__ import annotations
 
+import contextlib
 import math
 import sys
 import time
@@ -159,7 +160,9 @@ def _plain_row_norm(norm) -> bool:
     return layer_ops.plain_module(norm, RMSNorm) or layer_ops.plain_module(norm, hf)
 
 
-CAPTURE_FREE = 4 << 30  # device memory that a step's capture is sure to fit in
+# Free device memory below which a capture begins with the allocator's cached
+# blocks given back: HIP's own allocations for a graph cannot ask for them.
+CAPTURE_FREE = 4 << 30
 
 
 @dataclass
@@ -607,19 +610,32 @@ class LlamaPagedDecodeRunner:
             self._staged = None
 
     def _capture(self, st: "_StepBuffers", side: torch.cuda.Stream) -> torch.cuda.CUDAGraph:
-        """The step captured on the stream its eager run warmed up. Cached
-        device memory is given back first only where less than CAPTURE_FREE
-        is left: it takes 3 ms, and the next prefill allocates it anew."""
+        """The step captured on the stream its eager run warmed up. The
+        allocator gives no cached block back while a capture is underway, so
+        one that runs out of memory is made again with all of them given
+        back. Before every capture would take 3 ms, and the next prefill
+        allocates the blocks anew."""
         torch.cuda.synchronize(self.device)
         if torch.cuda.mem_get_info(self.device)[0] < CAPTURE_FREE:
             torch.cuda.empty_cache()
+        try:
+            return self._record(st, side)
+        except torch.OutOfMemoryError:
+            pass  # the failed capture's own blocks go with the exception
+        torch.cuda.empty_cache()
+        return self._record(st, side)
+
+    def _record(self, st: "_StepBuffers", side: torch.cuda.Stream) -> torch.cuda.CUDAGraph:
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.stream(side):
             graph.capture_begin()
             try:
                 self._graph_body(st)
-            finally:
-                graph.capture_end()
+            except BaseException:
+                with contextlib.suppress(RuntimeError):  # the body's own error is the one to see
+                    graph.capture_end()
+                raise
+            graph.capture_end()
         return graph
 
     def _graph_body(self, st: "_StepBuffers") -> None:
