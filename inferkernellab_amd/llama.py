@@ -182,7 +182,11 @@ class _StepBuffers:
 
 @dataclass(frozen=True)
 class LlamaPagedRunResult:
-    """Outcome and timing of a Llama run (fields of hf_benchmark.py:88-128)."""
+    """Outcome and timing of a Llama run (fields of hf_benchmark.py:88-128).
+
+    A captured step's logits are copied into the result while the next step
+    runs, so that copy is in the next step's time (the last one in its own):
+    the steps' sum and TPOT hold all of them, TTFT none."""
 
     backend: str
     append_backend: str
@@ -696,6 +700,8 @@ class LlamaPagedDecodeRunner:
                 t0 = time.perf_counter()
                 batch = self.runtime.step()
                 torch.cuda.synchronize(self.device)
+                if not (self.runtime.scheduler.waiting or self.runtime.scheduler.running):
+                    self._collect_logits()  # no step follows to take them
                 ms = (time.perf_counter() - t0) * 1e3
                 peak_blocks = max(peak_blocks, self.cache.allocator.num_used_blocks)
                 if batch.phase == "prefill":
@@ -704,7 +710,6 @@ class LlamaPagedDecodeRunner:
                     decode_steps.append(ms)
                 else:
                     raise RuntimeError("scheduler became idle before all requests finished")
-        self._collect_logits()
         if len(self._prompt_logits) != len(self.requests):
             raise RuntimeError("prefill did not produce one final logits tensor per request")
         generated = tuple(tuple(self._generated[r.request_id]) for r in self.requests)

@@ -436,3 +436,29 @@ def test_llama_graph_decode_equals_eager_decode():
     for a, b in zip(runs[0].decode_logits, runs[1].decode_logits):
         assert torch.equal(a, b)
     assert runs[0].cache_released
+
+
+def test_llama_step_times_hold_every_copy_of_the_logits(monkeypatch):
+    """A captured step's logits are taken into the result under the next step,
+    the last step's within its own time: slowed down, each shows in the sum."""
+    import time
+
+    from inferkernellab_amd.llama import LlamaConfig, LlamaPagedDecodeRunner, random_llama
+
+    cfg = LlamaConfig(vocab_size=128, hidden_size=256, intermediate_size=512, num_hidden_layers=1,
+                      num_attention_heads=4, num_key_value_heads=2)
+    runner = LlamaPagedDecodeRunner(random_llama(cfg, seed=1, device="cuda", dtype=torch.float32), [[1, 2, 3]],
+                                    max_new_tokens=3)
+    collect, taken = runner._collect_logits, []
+
+    def slow_collect():
+        if runner._staged is not None:
+            time.sleep(0.2)
+            taken.append(1)
+        collect()
+
+    monkeypatch.setattr(runner, "_collect_logits", slow_collect)
+    result = runner.run()
+    assert len(taken) == len(result.decode_logits) == 3
+    # the first step holds its eager run and the capture, and no copy
+    assert result.decode_step_wall_ms[1] >= 200 and result.decode_step_wall_ms[2] >= 400
