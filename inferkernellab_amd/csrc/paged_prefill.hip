@@ -711,7 +711,8 @@ extern "C" int32_t ikl_paged_prefill_path(int32_t dtype, int32_t head_dim, int32
 
 extern "C" int32_t ikl_paged_prefill_plan(const ikl_paged_prefill_args *a, int64_t longest_context,
                                           int64_t shortest_start) {
-  if (!a || a->batch <= 0 || a->query_width <= 0 || a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0 ||
+  if (!a || a->batch <= 0 || a->query_width <= 0 || a->num_heads <= 0 || a->num_kv_heads <= 0 ||
+      a->num_heads % a->num_kv_heads != 0 || a->head_dim <= 0 || a->block_size <= 0 || a->table_width <= 0 ||
       longest_context < 0 || shortest_start < 0)
     return fail(IKL_EINVAL, "ikl_paged_prefill_plan: invalid arguments");
   const int path = a->path == IKL_PATH_SCALAR_GROUPED ? a->path

@@ -105,3 +105,14 @@ def test_invalid_ranges_are_refused():
     a = _args(1, 8, 2, 64, 16, 8)
     assert _plan(a, -1, 0) == _lib.IKL_EINVAL and _plan(a, 16, -1) == _lib.IKL_EINVAL
     assert _lib.load().ikl_paged_prefill_plan(None, 0, 0) == _lib.IKL_EINVAL
+
+
+@pytest.mark.parametrize("name", ["batch", "query_width", "num_heads", "num_kv_heads", "head_dim", "block_size",
+                                  "table_width"])
+@pytest.mark.parametrize("value", [0, -16])
+def test_invalid_sizes_are_refused(name, value):
+    a = _args(1, 8, 2, 64, 16, 8)
+    setattr(a, name, value)
+    lib = _lib.load()
+    assert _plan(a, 16, 0) == _lib.IKL_EINVAL
+    assert lib.ikl_paged_prefill_key_groups(ctypes.byref(a)) == _lib.IKL_EINVAL
