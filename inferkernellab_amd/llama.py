@@ -22,6 +22,7 @@ to the activation dtype) for seeded random-weight models.
 from __future__ import annotations
 
 import contextlib
+import gc
 import math
 import sys
 import time
@@ -158,6 +159,20 @@ def _plain_row_norm(norm) -> bool:
     sees the call: RMSNorm here, or Transformers' where that is loaded."""
     hf = getattr(sys.modules.get("transformers.models.llama.modeling_llama"), "LlamaRMSNorm", RMSNorm)
     return layer_ops.plain_module(norm, RMSNorm) or layer_ops.plain_module(norm, hf)
+
+
+@contextlib.contextmanager
+def _collection_held_off():
+    """No automatic garbage collection inside. Collecting a dead graph calls
+    HIP, which refuses it during a capture; the error leaves a destructor and
+    ends the process."""
+    enabled = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if enabled:
+            gc.enable()
 
 
 # Free device memory below which a capture begins with the allocator's cached
@@ -631,7 +646,7 @@ class LlamaPagedDecodeRunner:
 
     def _record(self, st: "_StepBuffers", side: torch.cuda.Stream) -> torch.cuda.CUDAGraph:
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.stream(side):
+        with torch.cuda.stream(side), _collection_held_off():
             graph.capture_begin()
             try:
                 self._graph_body(st)
@@ -695,21 +710,27 @@ class LlamaPagedDecodeRunner:
         # otherwise create torch's graph-safe generator state as inference
         # tensors, and any later capture in the process outside inference
         # mode would fail on it
-        with torch.no_grad():
-            while self.runtime.scheduler.waiting or self.runtime.scheduler.running:
-                t0 = time.perf_counter()
-                batch = self.runtime.step()
-                torch.cuda.synchronize(self.device)
-                if not (self.runtime.scheduler.waiting or self.runtime.scheduler.running):
-                    self._collect_logits()  # no step follows to take them
-                ms = (time.perf_counter() - t0) * 1e3
-                peak_blocks = max(peak_blocks, self.cache.allocator.num_used_blocks)
-                if batch.phase == "prefill":
-                    prefill_steps.append(ms)
-                elif batch.phase == "decode":
-                    decode_steps.append(ms)
-                else:
-                    raise RuntimeError("scheduler became idle before all requests finished")
+        try:
+            with torch.no_grad():
+                while self.runtime.scheduler.waiting or self.runtime.scheduler.running:
+                    t0 = time.perf_counter()
+                    batch = self.runtime.step()
+                    torch.cuda.synchronize(self.device)
+                    if not (self.runtime.scheduler.waiting or self.runtime.scheduler.running):
+                        self._collect_logits()  # no step follows to take them
+                    ms = (time.perf_counter() - t0) * 1e3
+                    peak_blocks = max(peak_blocks, self.cache.allocator.num_used_blocks)
+                    if batch.phase == "prefill":
+                        prefill_steps.append(ms)
+                    elif batch.phase == "decode":
+                        decode_steps.append(ms)
+                    else:
+                        raise RuntimeError("scheduler became idle before all requests finished")
+        finally:
+            # The runner and its runtime refer to each other: left to the
+            # garbage collector, the graphs would die at any later moment,
+            # another capture included.
+            self._graphs.clear()
         if len(self._prompt_logits) != len(self.requests):
             raise RuntimeError("prefill did not produce one final logits tensor per request")
         generated = tuple(tuple(self._generated[r.request_id]) for r in self.requests)

@@ -1,8 +1,11 @@
 """Capturing a decode step when memory runs out: the capture is made again once
 the allocator has given its cached blocks back, those of the failed capture
-included, and any other error is the caller's."""
+included, and any other error is the caller's. And that no graph is destroyed
+during a capture, which would end the process: no garbage is collected in one,
+and a run leaves no graph to the collector."""
 
 import contextlib
+import gc
 import weakref
 
 import pytest
@@ -63,6 +66,58 @@ def test_a_second_failure_and_other_errors_are_raised(device):
     with pytest.raises(ValueError, match="wrong"):
         _runner([(ValueError, "wrong")])._capture(None, None)
     assert [x for x in device if not isinstance(x, weakref.ref)] == ["begin", "end"]
+
+
+@pytest.mark.parametrize("enabled", [True, False])
+@pytest.mark.parametrize("error", [None, ValueError])
+def test_no_garbage_is_collected_during_a_capture(device, enabled, error):
+    class Cycle:
+        def __init__(self):
+            self.me = self
+
+    before = gc.isenabled()
+    (gc.enable if enabled else gc.disable)()
+    try:
+        runner, collected = _runner([]), []
+
+        def body(st):
+            dead = Cycle()
+            weakref.finalize(dead, collected.append, 1)
+            del dead
+            garbage = [[] for _ in range(200_000)]  # far past the collector's thresholds
+            assert garbage and not collected
+            if error is not None:
+                raise error("body")
+
+        runner._graph_body = body
+        with pytest.raises(error) if error else contextlib.nullcontext():
+            runner._capture(None, None)
+        assert gc.isenabled() == enabled
+    finally:
+        (gc.enable if before else gc.disable)()
+
+
+@pytest.mark.gpu
+def test_a_run_leaves_no_graph_behind(monkeypatch):
+    cfg = LlamaConfig(vocab_size=128, hidden_size=256, intermediate_size=512, num_hidden_layers=1,
+                      num_attention_heads=4, num_key_value_heads=2)
+    runner = LlamaPagedDecodeRunner(random_llama(cfg, seed=3, device="cuda", dtype=torch.float32),
+                                    [[1, 2, 3], [4, 5]], max_new_tokens=3)
+    graphs, record = [], runner._record
+
+    def recorded(st, side):
+        graph = record(st, side)
+        graphs.append(weakref.ref(graph))
+        return graph
+
+    monkeypatch.setattr(runner, "_record", recorded)
+    gc.disable()
+    try:
+        result = runner.run()
+        assert graphs and all(g() is None for g in graphs)
+    finally:
+        gc.enable()
+    assert len(result.decode_logits) == 3
 
 
 @pytest.mark.gpu
