@@ -14,6 +14,7 @@ import ctypes
 
 import torch
 from torch import nn
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from .ops import _DTYPES, _on_device, _require_backend
@@ -42,15 +43,24 @@ def plain_module(module, cls) -> bool:
     return type(module) is cls and unhooked(module)
 
 
+def unwatched() -> bool:
+    """True when no dispatch or function mode sees torch's calls (a flop
+    counter, a tracer, a replacement for F.linear). A default device is a
+    function mode too, and sees only what makes new tensors."""
+    modes = (torch._C._get_function_stack_at(i) for i in range(torch._C._len_torch_function_stack()))
+    return torch._C._len_torch_dispatch_stack() == 0 and all(type(m) is DeviceContext for m in modes)
+
+
 def kernels_apply(x: torch.Tensor) -> bool:
     """Whether a module call on `x` may be restated by a kernel at all: no
-    graph to record, no autocast, a plain tensor on a GPU."""
+    graph to record, no autocast, nobody watching, a plain tensor on a GPU."""
     return (
         type(x) is torch.Tensor
         and x.device.type == "cuda"
         and x.dtype in _DTYPES
         and not torch.is_grad_enabled()
         and not torch.is_autocast_enabled()
+        and unwatched()
     )
 
 

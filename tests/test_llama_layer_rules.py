@@ -1,8 +1,8 @@
 """Which layers of a decode step the linear kernels restate: they read the
 norms' output in the norm kernel's own layout, so a norm that runs as a module
 (any type, any strides may come out of it) takes the whole layer to its
-modules. And which final norms and heads a prefill gives the chunks' last rows
-alone. The rules themselves run here, with the device condition stubbed."""
+modules. No kernel stands in for a module while a mode watches torch's calls.
+And which final norms and heads a prefill gives the chunks' last rows alone. The rules themselves run here, with the device condition stubbed."""
 
 import pytest
 import torch
@@ -51,6 +51,29 @@ def test_norm_that_runs_as_a_module_keeps_the_layers_linears(layer, name, change
 
 def test_delta_that_promotes_the_residual_keeps_the_layers_linears(layer):
     assert not _restated(layer, torch.zeros(3, 64))
+
+
+class _GpuLooking:
+    """A plain tensor on a GPU, to the rule."""
+
+    device, dtype = torch.device("cuda"), torch.bfloat16
+
+
+def test_a_watched_call_is_left_to_the_module(monkeypatch):
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+
+    monkeypatch.setattr(layer_ops.torch, "Tensor", _GpuLooking)
+    x = _GpuLooking()
+    with torch.no_grad():
+        assert layer_ops.kernels_apply(x)
+        with torch.device("cpu"):  # a default device is no watcher
+            assert layer_ops.kernels_apply(x)
+        with TorchFunctionMode():
+            assert not layer_ops.kernels_apply(x)
+        with FlopCounterMode(display=False):
+            assert not layer_ops.kernels_apply(x)
+        assert layer_ops.kernels_apply(x)
 
 
 class _RecordingNorm(RMSNorm):
