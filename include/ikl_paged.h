@@ -268,8 +268,8 @@ typedef struct ikl_paged_prefill_args {
 int ikl_paged_prefill_attention(const ikl_paged_prefill_args *args, void *stream);
 
 /* How a prefill launch runs. On the matrix-core path: 1, 2 or 4 waves share
- * each row (launches that leave the chip idle), 0 when all waves of a
- * workgroup walk the keys together. On the other path: IKL_PREFILL_ROWS for
+ * each row (launches of long contexts that leave the chip idle), 0 when all
+ * waves of a workgroup walk the keys together. On the other path: IKL_PREFILL_ROWS for
  * one wave per row (short contexts, wide rows), 0 for the fp32 matrix cores.
  * longest_context /
  * shortest_start: the largest element of context_lens and the smallest of

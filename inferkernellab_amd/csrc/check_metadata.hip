@@ -101,7 +101,7 @@ extern "C" int32_t ikl_check_metadata(const void *tables, int32_t table_type, in
   p.table_i64 = table_type == IKL_I64;
   p.lens_i64 = lens_type == IKL_I64;
   p.flags = flags;
-  // a workgroup per 16 segments, four waves' loads each twice over
+  // a workgroup per 16 segments: two for each of its eight waves
   const int64_t want = (batch * p.segs + 2 * CHECK_WAVES - 1) / (2 * CHECK_WAVES);
   const int32_t grid = (int32_t)(want < num_flags ? want : num_flags);
   for (int32_t i = 0; i < grid; ++i) reinterpret_cast<volatile uint32_t *>(flags)[i] = IKL_CHECK_PENDING;

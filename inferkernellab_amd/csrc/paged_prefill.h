@@ -55,7 +55,7 @@ constexpr int PREFILL_F32_MAX_DIM = 256;
 hipError_t launch_prefill_f32(PrefillParams p, int dtype, hipStream_t s);
 
 // Launches paged_prefill_split_kernel (what the 16-bit kernel takes) with
-// `groups` (2 or 4) waves on every row; p.row_blocks and p.bh_pad are set
+// `groups` (1, 2 or 4) waves on every row; p.row_blocks and p.bh_pad are set
 // here.
 hipError_t launch_prefill_split(PrefillParams p, int dtype, int groups, hipStream_t s);
 

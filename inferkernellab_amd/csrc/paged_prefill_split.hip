@@ -1,4 +1,5 @@
-// Paged prefill for launches that leave the chip idle: the shapes and results
+// Paged prefill for launches of long contexts that leave the chip idle (the
+// rule is prefill_key_groups in paged_prefill.hip): the shapes and results
 // of paged_prefill_mfma_kernel (paged_prefill.hip), where a workgroup's 4
 // waves own 128 rows and walk the keys together. There few rows over long
 // prefixes are few workgroups, each a serial chain of all its key tiles, and
@@ -14,9 +15,10 @@
 // favours few instructions (32x32x16 MFMAs: half as many, one softmax row per
 // lane, 8 dot products for the denominators) and runs the next tile's QK^T
 // under this one's exponentials. 9 % fewer cycles than the 16x16x32 loop on
-// the ragged chunks below. At 8 x 4096 it is 6.5 % fewer (2.69 -> 2.52 M), but
-// that launch meets the power limit: the clock falls from 2155 to 2042 MHz
-// and it takes 1173-1206 us against 1160, which is why the other kernel stays.
+// the ragged chunks below. At 8 x 4096 it is 6 % fewer (2.68 -> 2.52 M), but
+// that launch meets the power limit: the clock falls from 2219-2226 to
+// 2000-2040 MHz and it takes 1234-1260 us against 1201-1207 (medians of two
+// counter runs), which is why the other kernel stays.
 //
 // 32/8 heads of 128, bf16, against paged_prefill_mfma_kernel: 4 requests x
 // (2000 + 64 tokens) 57.6 -> 28.9 us, 1 x 1024 tokens 32.1 -> 23.8, 2 x 1024
