@@ -17,8 +17,9 @@
  *     (cache.k[layer], cache.v[layer]) plus its block/token/head strides.
  *   - The last dimension (head_dim) of every tensor is contiguous.
  *   - All work is enqueued on `stream` (a hipStream_t, NULL = default
- *     stream). No call synchronises the host, allocates device memory or
- *     keeps device state between calls.
+ *     stream). No call synchronises the host (ikl_check_metadata_wait is
+ *     there to wait), allocates device memory or keeps device state
+ *     between calls.
  *   - Return value: 0 on success, a negative IKL_E* code otherwise; the
  *     message of the last failure on the calling thread is returned by
  *     ikl_last_error().
